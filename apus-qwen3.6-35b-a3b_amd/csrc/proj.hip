@@ -18,9 +18,12 @@
 //                tile, its operands copied global -> LDS by buffer_load ...
 //                lds in stages of 32 k through a 4-deep ring; each
 //                wavefront reads the next k16 step's fragments while the
-//                current step's MFMAs issue. Tile shapes are chosen per call
-//                shape (decode batches: small tiles, many workgroups;
-//                prefill: 256 x 256). It sums in its own order: the
+//                current step's MFMAs issue.
+//   k_gemm_wide  the same product with one wavefront per SIMD, for calls
+//                with enough tiles to fill the chip. The tile shape (and
+//                with it the kernel) is the one with the least estimated
+//                time; every shape accumulates an element's k16 steps in
+//                the same order. They sum in their own order: the
 //                tolerance class of the attention kernels (|c - r| <=
 //                2e-3 (|r| + esc), esc = sum_k |w x|).
 // Host-pointer drop-ins keep device copies of the weights keyed by their
@@ -167,44 +170,34 @@ __device__ __forceinline__ int tile_slot(int r, int c) { return r * 64 + ((c ^ (
 constexpr int kTileStages = 4;            // LDS ring depth (stages of 32 k)
 
 // Workgroup -> (output tile, row tile). Workgroups are dealt round-robin
-// to the 8 XCDs (id % 8), each XCD running its ids in order. The tiles are
-// grouped into blocks of GO output tiles x GM row tiles (GO GM = 32, GM =
-// 8 for 8 or more row tiles); block g goes to XCD g % 8 as its (g / 8)-th group of
-// 32 ids. The 32 workgroups an XCD runs together then share GO weight
-// tiles and GM x tiles, which stay in that XCD's L2 while they walk K in
-// step (prefill: 12 distinct 256-row operand tiles per XCD instead of 18
-// with whole row-tile columns per XCD).
-__host__ __device__ inline void tile_groups(int nbo, int nbm, int &go, int &gm, int &ngo,
-                                            int &ngm) {
-    gm = nbm < 8 ? nbm : 8;
-    go = 32 / gm;
-    ngo = (nbo + go - 1) / go;
-    ngm = (nbm + gm - 1) / gm;
-}
-// Fewer than 8 row tiles (decode batches): output tile ob's row tiles all
-// go to XCD ob % 8 instead (ids ((ob / 8) nbm + mb) 8 + ob % 8), which
-// measured faster there (w_out at 325 rows: 27 vs 29 us).
-__host__ __device__ inline int tile_grid(int nbo, int nbm) {
-    if (nbm < 8) return (nbo + 7) / 8 * 8 * nbm;
-    int go, gm, ngo, ngm;
-    tile_groups(nbo, nbm, go, gm, ngo, ngm);
-    return (ngo * ngm + 7) / 8 * 8 * 32;
-}
+// to the 8 XCDs (id % 8), each XCD running its ids in order, so XCD x gets
+// tiles x q .. x q + q - 1 (q an eighth of the tiles) of an order in which
+// the 32 tiles that an XCD runs together share operand tiles, which stay in
+// that XCD's L2 while they walk K in step: with 8 or more row tiles, blocks
+// of 4 output x 8 row tiles (12 distinct operand tiles instead of 18 with
+// whole row-tile columns); with fewer, an output tile's row tiles one after
+// the other. Every XCD has the same number of tiles to within one (whole
+// 4 x 8 blocks dealt to XCDs left half of the chip idle below 8 blocks:
+// 2048 outputs x 512 rows, K = 4096, 34.7 us, now 17.4).
+__host__ __device__ inline int tile_grid(int nbo, int nbm) { return (nbo * nbm + 7) / 8 * 8; }
 __host__ __device__ inline void tile_of(int id, int nbo, int nbm, int &ob, int &mb) {
-    if (nbm < 8) {
-        const int band = id / (8 * nbm), rem = id % (8 * nbm);
-        mb = rem / 8;
-        ob = band * 8 + rem % 8;
+    const int n = nbo * nbm, q = (n + 7) / 8, t = (id % 8) * q + id / 8;
+    if (t >= n) {
+        ob = nbo;                                  // past the last tile
+        mb = 0;
         return;
     }
-    int go, gm, ngo, ngm;
-    tile_groups(nbo, nbm, go, gm, ngo, ngm);
-    const int x = id % 8, slot = id / 8;
-    const int g = (slot / 32) * 8 + x, p = slot % 32;
-    const int gi = g / ngm, gj = g % ngm;          // group (output, row)
-    ob = gi * go + p % go;
-    mb = gj * gm + p / go;
-    if (gi >= ngo) ob = nbo;                       // past the last group
+    if (nbm < 8) {
+        ob = t / nbm;
+        mb = t % nbm;
+        return;
+    }
+    // bands of 8 row tiles; in a band, blocks of 4 output tiles, row fastest
+    const int band = t / (8 * nbo), rows = min(8, nbm - 8 * band);
+    const int p = t - 8 * nbo * band;
+    const int blk = p / (4 * rows), w = min(4, nbo - 4 * blk), e = p - 4 * rows * blk;
+    ob = 4 * blk + e % w;
+    mb = 8 * band + e / w;
 }
 
 __device__ __forceinline__ int seg_of(const GemmSegs &g, int o) {
@@ -414,16 +407,260 @@ __global__ __launch_bounds__(64 * WO * WM) void k_gemm_tile(GemmSegs sg,
     store_tiles<TO, TMM>(sg, acc, o0 + wo * TO * 32, m0 + wm * TMM * 32, O, M, lane);
 }
 
-// Decode-sized row counts: one BO x BM tile per workgroup (BO = 32 TO
-// outputs, BM = 32 TMM rows), its NW wavefronts each over a contiguous
-// 1/NW share of the k stages. Each wavefront copies its own stages into a
-// private R-deep LDS ring (the same 1 KiB pieces and swizzle as
-// k_gemm_tile) and waits only for its own copies: no barrier in the k loop,
-// where the shared-ring kernel's per-stage barrier left a decode tile's
-// two wavefronts waiting on each other for every 32 k. The NW partial
-// tiles are then summed through LDS in a fixed tree (NW = 4: (p0 + p2) +
-// (p1 + p3), p_w the partial of share w), and wavefront 0 stores the
-// tile. An element's sum order depends on K and NW only.
+// ---- k_gemm_wide ---------------------------------------------------------
+// The same product, operands and summation order as k_gemm_tile (bitwise
+// the same result), with 4 wavefronts (2 x 2), one per SIMD, of TO x TMM
+// MFMA tiles each. What bounded k_gemm_tile at 256 x 256 (8 wavefronts of
+// 4 x 2 tiles, 32-k stages) and what changed here, on a 2048 x 8192 x 4096
+// product, 256 tiles, in us per 32 k (the MFMAs alone: 0.59):
+//   0.95  as it was. 64-byte half lines per row and copy, and a wavefront
+//         reads 6 fragments from LDS for 8 MFMAs;
+//   0.87  4 x 4 tiles (8 reads for 16 MFMAs), 64-k stages, so that a copy
+//         reads whole 128-byte lines;
+//   0.77  each line touched once per XCD a stage before its copies: the
+//         workgroups of an XCD walk K in step, so each stage's lines all
+//         missed L2 together, and a stage was a trip to HBM long.
+// The stores of a tile go through LDS as whole rows (what a call takes
+// besides its k steps: 23 -> 7 us). 4096 x 12352 x 2048: 236 -> 201 us (1.03
+// PFLOP/s).
+constexpr int kWideK = 64;                // k per stage
+
+// 16 (4) bytes per lane from a 64-bit address to LDS byte lds + 16 (4) *
+// lane. The addresses are VGPRs: a buffer resource per copy piece would
+// need more SGPRs than there are. The s_nop is the wait state between a
+// write of M0 and its use here. live: all ones, or zero for a copy that
+// counts as issued (vmcnt) but moves nothing; the wavefront's lanes are all
+// active here.
+__device__ __forceinline__ void dma16_g(const char *p, uint32_t lds, int live) {
+    lds = __builtin_amdgcn_readfirstlane(lds);
+    live = __builtin_amdgcn_readfirstlane(live);
+    asm volatile("s_mov_b32 exec_lo, %2\n\ts_mov_b32 exec_hi, %2\n\t"
+                 "global_load_lds_dwordx4 %0, off\n\ts_mov_b64 exec, -1"
+                 ::"v"(p), "{m0}"(lds), "s"(live) : "memory");
+}
+__device__ __forceinline__ void dma4_g(const char *p, uint32_t lds) {
+    lds = __builtin_amdgcn_readfirstlane(lds);
+    asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(p), "{m0}"(lds) : "memory");
+}
+
+// Tile (o0, m0) of 64 TO outputs x 64 TMM rows. sw workgroups of this XCD
+// share its w rows (this one is number iw of them), 32 / sw its x rows
+// (number ix). A stage in LDS: BO w rows, then BM x rows, of 128 bytes;
+// 16-byte chunk c of row r at slot c ^ (r % 8), so that the 8 rows of one
+// LDS read phase hit 8 distinct slots. K is a multiple of 32: an odd last
+// half stage has no second half to read, so its copies repeat the first.
+template <int TO, int TMM>
+__device__ __forceinline__ void gemm_wide(char *sm, const GemmSegs &sg, const uint16_t *x, int M,
+                                          int K, int o0, int m0, int sw, int iw, int ix) {
+    constexpr int NW = 4, BO = 64 * TO, BM = 64 * TMM;
+    constexpr int PB = BO * 128, SB = (BO + BM) * 128;
+    constexpr int PPW = (BO + BM) / 8 / NW, NF = TO * TMM, NR = TO + TMM;
+    static_assert((BO + BM) / 8 % NW == 0, "copy pieces must split evenly over the wavefronts");
+    const int O = sg.row0[sg.n];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wo = wave >> 1, wm = wave & 1;
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_void *)sm);
+    const int nk = (K + kWideK - 1) / kWideK;
+    const bool odd = K % kWideK != 0;
+    // this wavefront's copy pieces: 8 rows of 128 bytes each, in one
+    // segment. Rows past O or M read the last row (their products are not
+    // stored).
+    const char *src[PPW];
+    const int cg = (lane & 7) ^ (lane >> 3);               // chunk: slot ^ row % 8
+    // the last stage's step back to its first half
+    const int tail = odd && cg >= 4 ? -64 : 0;
+#pragma unroll
+    for (int i = 0; i < PPW; i++) {
+        const int p = wave * PPW + i;
+        const bool pw = p < BO / 8;
+        const int ob = min(o0 + p * 8, O - 1), si = __builtin_amdgcn_readfirstlane(seg_of(sg, ob));
+        const uint16_t *base = pw ? sg.w[si] : x;
+        const int r = p * 8 + (lane >> 3);
+        const int row = pw ? min(o0 + r, O - 1) - sg.row0[si] : min(m0 + r - BO, M - 1);
+        src[i] = (const char *)(base + (size_t)row * K) + cg * 16 + (nk == 1 ? tail : 0);
+    }
+    const uint32_t piece0 = lds0 + wave * PPW * 1024;
+    // copy i of the stage in flight into ring slot `slot`; its address then
+    // moves on by adv, to the next stage
+    auto copy = [&](int i, uint32_t slot, int adv, int live) {
+        dma16_g(src[i], piece0 + slot + i * 1024, live);
+        src[i] += adv;
+    };
+    // from stage st to st + 1 (past the last stage it stays)
+    auto advance = [&](int st) { return st + 1 < nk ? 128 + (st + 2 == nk ? tail : 0) : 0; };
+    // Prefetch into L2: this workgroup's share of the lines of its operand
+    // tiles, one 4-byte load per line into an LDS row that nothing reads.
+    // Every lane loads, so that the wait counts are the same in every
+    // wavefront.
+    const char *pf;
+    {
+        const int nw = (BO + sw - 1) / sw, sx = 32 / sw, nx = (BM + sx - 1) / sx;
+        const int e = threadIdx.x;
+        const bool px = e >= nw && e < nw + nx;
+        const int o = min(o0 + iw * nw + (e < nw ? e : 0), O - 1), si = seg_of(sg, o);
+        const int row = px ? min(m0 + ix * nx + e - nw, M - 1) : o - sg.row0[si];
+        pf = (const char *)((px ? x : sg.w[si]) + (size_t)row * K) + min(2, nk - 1) * 128;
+    }
+    auto prefetch = [&](int st) {            // stages 2, 3, ... in turn
+        dma4_g(pf, lds0 + 2 * SB + wave * 256);
+        pf += st + 1 < nk ? 128 : 0;
+    };
+    f32x16 acc[TO][TMM];
+#pragma unroll
+    for (int t = 0; t < TO; t++)
+#pragma unroll
+        for (int u = 0; u < TMM; u++) acc[t][u] = f32x16{};
+    struct Frag {
+        bf16x8 a[TO], b[TMM];
+    };
+    // chunk 2 s + lane / 32 of row lane % 32 of a 32-row block, s = 0
+    const uint32_t rbase = (lane & 31) * 128 + (((lane >> 5) ^ (lane & 7)) << 4);
+    // operand read j of k16 step s of the stage in `slot`, in the order the
+    // MFMAs use them: a[0], b[0..], a[1..]
+    auto rd1 = [&](uint32_t slot, int s, int j, Frag &f) {
+        const char *p = sm + ((rbase ^ (s << 5)) + slot);
+        if (j == 0 || j > TMM) {
+            const int t = j == 0 ? 0 : j - TMM;
+            f.a[t] = *reinterpret_cast<const bf16x8 *>(p + wo * TO * 4096 + t * 4096);
+        } else {
+            f.b[j - 1] = *reinterpret_cast<const bf16x8 *>(p + PB + wm * TMM * 4096 + (j - 1) * 4096);
+        }
+    };
+    using no = std::false_type;
+    using yes = std::true_type;
+    // One k16 step: its NF MFMAs on f and, fenced in place between them, the
+    // reads of the next step's operands into g (READ: k16 step s2 of slot
+    // rslot) and the copies of a stage into cslot (COPY).
+    auto step = [&](const Frag &f, Frag &g, auto read, uint32_t rslot, int s2, auto cpy,
+                    uint32_t cslot, int adv, int live) {
+        constexpr bool READ = decltype(read)::value, COPY = decltype(cpy)::value;
+        int r = 0, d = 0;
+#pragma unroll
+        for (int i = 0; i < NF; i++) {
+            acc[i / TMM][i % TMM] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                f.a[i / TMM], f.b[i % TMM], acc[i / TMM][i % TMM], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            // the reads go under the first three quarters of the MFMAs
+#pragma unroll
+            for (; READ && r < NR && (i == NF - 1 || r * NF * 3 <= i * NR * 4); r++) rd1(rslot, s2, r, g);
+#pragma unroll
+            for (; COPY && d < PPW && d * NF < (i + 1) * PPW; d++) copy(d, cslot, adv, live);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    Frag f0, f1;
+    // stages 0 and 1 in flight; stage 0 published
+    const int adv0 = advance(0), adv1 = advance(1);
+#pragma unroll
+    for (int i = 0; i < PPW; i++) copy(i, 0, adv0, -1);
+#pragma unroll
+    for (int i = 0; i < PPW; i++) copy(i, SB, adv1, (1 - nk) >> 31);
+    prefetch(2);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PPW + 1) : "memory");
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NR; j++) rd1(0, 0, j, f0);
+    uint32_t slot = 0;
+    for (int kt = 0; kt < nk - 1; kt++) {
+        step(f0, f1, yes{}, slot, 1, no{}, 0, 0, 0);
+        step(f1, f0, yes{}, slot, 2, no{}, 0, 0, 0);
+        step(f0, f1, yes{}, slot, 3, no{}, 0, 0, 0);
+        // every operand of this stage has been read, by this wavefront (it
+        // waited for f1) and after the barrier by all, and the next stage has
+        // landed (its copies are older than the last prefetch): stage
+        // kt + 2 goes into this stage's slot
+        asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
+        __syncthreads();
+        step(f1, f0, yes{}, slot ^ SB, 0, yes{}, slot, advance(kt + 2), (kt + 2 - nk) >> 31);
+        prefetch(kt + 3);
+        slot ^= SB;
+    }
+    // the last stage; an odd K's second half is zeros
+    auto mask = [&](Frag &f) {
+        if (!odd) return;
+#pragma unroll
+        for (int t = 0; t < TO; t++) f.a[t] = bf16x8{};
+#pragma unroll
+        for (int u = 0; u < TMM; u++) f.b[u] = bf16x8{};
+    };
+    step(f0, f1, yes{}, slot, 1, no{}, 0, 0, 0);
+    step(f1, f0, yes{}, slot, 2, no{}, 0, 0, 0);
+    mask(f0);
+    step(f0, f1, yes{}, slot, 3, no{}, 0, 0, 0);
+    mask(f1);
+    step(f1, f0, no{}, 0, 0, no{}, 0, 0, 0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();                     // the ring is free: no copy in flight, no reader
+    // Epilogue: lane -> m = lane % 32, o = 8 (i / 4) + 4 (lane / 32) + i % 4
+    // of each 32 x 32 tile. Through LDS (this wavefront's quarter, rows m of
+    // 64 TO bytes, 16-byte chunk c at c ^ (m % NCH)) so that the stores are
+    // 16-byte pieces of whole rows; a row stored straight from the
+    // accumulators would be 8-byte pieces of 32 rows per instruction.
+    const int ow = o0 + wo * TO * 32, mw = m0 + wm * TMM * 32;
+    bool vec = true;
+    for (int i = 0; i < sg.n; i++)
+        vec = vec && ((sg.ldy[i] | sg.row0[i] | sg.row0[i + 1]) & 7) == 0 && ((uintptr_t)sg.y[i] & 15) == 0;
+    if (!vec) {
+        store_tiles<TO, TMM>(sg, acc, ow, mw, O, M, lane);
+        return;
+    }
+    constexpr int NCH = 4 * TO, ROW = 64 * TO;           // chunks, bytes of a row
+    char *ep = sm + wave * (TMM * 32 * ROW);
+#pragma unroll
+    for (int t = 0; t < TO; t++)
+#pragma unroll
+        for (int u = 0; u < TMM; u++) {
+            const int m = u * 32 + (lane & 31);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const f32x16 &v = acc[t][u];
+                *reinterpret_cast<uint2 *>(ep + m * ROW + (((t * 4 + q) ^ (m & (NCH - 1))) << 4) +
+                                           ((lane >> 5) << 3)) =
+                    make_uint2(pk2(v[4 * q], v[4 * q + 1]), pk2(v[4 * q + 2], v[4 * q + 3]));
+            }
+        }
+    // (own quarter only: a wavefront's LDS accesses execute in order)
+    constexpr int RPI = 64 / NCH;                        // rows per instruction
+    const int pc = lane & (NCH - 1);
+    const int o = ow + pc * 8, si = seg_of(sg, min(o, O - 1));
+    uint16_t *yo = sg.y[si] + (o - sg.row0[si]);
+    const int ld = sg.ldy[si];
+#pragma unroll 8
+    for (int i = 0; i < TMM * 32 / RPI; i++) {
+        const int m = i * RPI + lane / NCH;
+        const uint4 v = *reinterpret_cast<const uint4 *>(ep + m * ROW + ((pc ^ (m & (NCH - 1))) << 4));
+        if (o < O && mw + m < M) *reinterpret_cast<uint4 *>(yo + (size_t)(mw + m) * ld) = v;
+    }
+}
+
+// A last output tile of at most 64 outputs (the GDN in-projection's gate
+// rows: 12352 = 48 * 256 + 64) runs as a 64-wide tile, ids after the
+// full tiles', instead of as a whole round of mostly empty 256-wide ones.
+template <int TO>
+__host__ __device__ inline bool wide_narrow(int O) { return TO == 4 && O % 256 > 0 && O % 256 <= 64 && O > 256; }
+
+template <int TO, int TMM>
+__global__ __launch_bounds__(256, TO * TMM <= 8 ? 2 : 1) void k_gemm_wide(
+    GemmSegs sg, const uint16_t *__restrict__ x, int M, int K) {
+    constexpr int BO = 64 * TO, BM = 64 * TMM;
+    __shared__ __attribute__((aligned(16))) char sm[2 * (BO + BM) * 128 + 1024];
+    const int O = sg.row0[sg.n];
+    const bool narrow = wide_narrow<TO>(O);
+    const int nbo = narrow ? O / BO : (O + BO - 1) / BO, nbm = (M + BM - 1) / BM;
+    const int n = tile_grid(nbo, nbm);
+    // the workgroups of this one's XCD that share its tiles (tile_of)
+    const int sw = min(nbm, 8);
+    if (TO == 4 && (int)blockIdx.x >= n) {
+        gemm_wide<1, TMM>(sm, sg, x, M, K, nbo * BO, ((int)blockIdx.x - n) * BM, 1, 0, 0);
+        return;
+    }
+    int ob, mb;
+    tile_of(blockIdx.x, nbo, nbm, ob, mb);
+    if (ob >= nbo) return;                      // (the grid is a multiple of 8)
+    gemm_wide<TO, TMM>(sm, sg, x, M, K, ob * BO, mb * BM, sw, mb % sw, ob % (32 / sw));
+}
+
 // y = rnd(sum over the splits of part, in split order), scattered to the
 // segments; a thread owns 4 consecutive outputs of one row (O % 4 == 0)
 __global__ __launch_bounds__(256) void k_gemm_reduce(GemmSegs sg, const float *__restrict__ part,
@@ -468,49 +705,73 @@ int launch_tile(const GemmSegs &sg, const uint16_t *x, int M, int K, const char 
     return kOk;
 }
 
+template <int TO, int TMM>
+int launch_wide(const GemmSegs &sg, const uint16_t *x, int M, int K, const char *name) {
+    constexpr int BO = 64 * TO, BM = 64 * TMM;
+    const int O = sg.row0[sg.n], nbm = (M + BM - 1) / BM;
+    const bool narrow = wide_narrow<TO>(O);
+    const unsigned grid = (unsigned)(tile_grid(narrow ? O / BO : (O + BO - 1) / BO, nbm) + (narrow ? nbm : 0));
+    APUS_TIMED(name, k_gemm_wide<TO, TMM><<<grid, 256, 0, stream()>>>(sg, x, M, K));
+    return launch_check(name);
+}
+
+// Tile shapes and what they take, in us for K = 2048 (it scales with K for
+// all of them), measured over 512 .. 12352 outputs x 16 .. 4096 rows: with
+// up to one workgroup per CU `one`, of which `fill` only when all CUs have
+// one (shared bandwidth); with two, `two` (the small shapes run 2 to 5
+// workgroups per CU side by side). Small shapes win while they leave no CU
+// with a second one, since a workgroup walks K alone; large ones move
+// fewer operand bytes per product.
+struct TileShape {
+    int bo, bm;
+    float one, fill, two;
+    bool split;                             // has a K-split form
+    int (*run)(const GemmSegs &, const uint16_t *, int, int, const char *, int);
+};
+template <int TO, int TMM>
+int run_wide(const GemmSegs &sg, const uint16_t *x, int M, int K, const char *nm, int) {
+    return launch_wide<TO, TMM>(sg, x, M, K, nm);
+}
+const TileShape kTileShapes[] = {
+    {64, 64, 12.7f, 0.0f, 20.5f, true, launch_tile<2, 1, 1, 2>},
+    {128, 64, 15.5f, 0.0f, 33.0f, true, launch_tile<2, 2, 2, 1>},
+    {128, 128, 24.0f, 6.5f, 50.0f, true, launch_tile<2, 4, 2, 1>},
+    {128, 128, 27.0f, 2.0f, 41.5f, false, run_wide<2, 2>},
+    {128, 192, 31.0f, 4.0f, 64.6f, false, run_wide<2, 3>},
+    {256, 192, 49.0f, 10.0f, 97.0f, false, run_wide<4, 3>},
+    {256, 256, 62.0f, 12.0f, 124.0f, false, run_wide<4, 4>},
+};
+
 }  // namespace
 
 namespace apus {
 
-// Tile shape per call shape (measured on MI355X for the model's projection
-// shapes, K = 2048 / 4096): decode batches want many small workgroups
-// (the weights stream once; x is re-read from L2), prefill the 256 x 256
-// tile (operand traffic M O K (1/BO + 1/BM) through L2).
-int gemm_tile_split(const GemmSegs &sg, const uint16_t *x, size_t M, size_t K, const char *nm,
-                    int cfg, int nsplit) {
-    const int m = (int)M, k = (int)K;
-    const size_t O = (size_t)sg.row0[sg.n];
-    if (nsplit > 1 && O % 4) nsplit = 1;
-    nsplit = std::max(1, std::min(nsplit, (int)(K / 32)));
-    if (cfg < 0)
-        cfg = M > 512 ? 3 : (M > 64 && O > 10000) ? 2 : (M > 64 && O > 4096) ? 1 : 0;
-    // Within a configuration the row tile follows M (measured on the
-    // model's shapes: the slowest workgroup sets the time, so a row tile
-    // that is mostly past M wastes its CU): M <= 128 with long outputs
-    // runs 128 x 128 tiles on 8 wavefronts (39 -> 31 us at M = 128), M <=
-    // 384 128 x 192 (the in-projection at M = 325: 42 -> 39 us), and
-    // decode rows past 64 with short outputs 128 x 64 (the out-projection
-    // at M = 325: 21 -> 19 us).
-    switch (cfg) {
-    case 3: return launch_tile<2, 4, 4, 2>(sg, x, m, k, nm, nsplit);      // 256 x 256
-    case 2:
-        if (m <= 128) return launch_tile<2, 4, 2, 1>(sg, x, m, k, nm, nsplit);   // 128 x 128
-        if (m <= 384) return launch_tile<2, 2, 2, 3>(sg, x, m, k, nm, nsplit);   // 128 x 192
-        return launch_tile<2, 2, 2, 4>(sg, x, m, k, nm, nsplit);                 // 128 x 256
-    case 1: return launch_tile<4, 1, 1, 4>(sg, x, m, k, nm, nsplit);      // 128 x 128
-    default:
-        if (m > 64) return launch_tile<2, 2, 2, 1>(sg, x, m, k, nm, nsplit);     // 128 x 64
-        return launch_tile<2, 1, 1, 2>(sg, x, m, k, nm, nsplit);                 // 64 x 64
-    }
-}
-
-// Decode-sized row counts with a long K (the output projections, K =
-// 4096) split K in two: twice the workgroups for the few output tiles
-// (w_out at 325 rows: 27 -> 21 us). The split depends on M and K only, so
-// a product's summation order is the same whichever launch (segmented or
-// not) computes it.
+// The shape with the least estimated time. Decode-sized row counts with a
+// long K (the output projections, K = 4096) split K in two: twice the
+// workgroups for the few output tiles (w_out at 325 rows: 27 -> 21 us). The
+// split depends on M and K only, and every shape accumulates an element's
+// k16 steps in order, so a product's result is the same whichever shape
+// and launch (segmented or not) computes it.
 int gemm_tile(const GemmSegs &sg, const uint16_t *x, size_t M, size_t K, const char *nm) {
-    return gemm_tile_split(sg, x, M, K, nm, -1, (M <= 512 && K >= 4096) ? 2 : 1);
+    const int O = sg.row0[sg.n], cus = cu_count();
+    const int nsplit = M <= 512 && K >= 4096 && O % 4 == 0 ? 2 : 1;
+    const TileShape *best = nullptr;
+    float tbest = 0.0f;
+    for (const TileShape &t : kTileShapes) {
+        if (nsplit > 1 && !t.split) continue;
+        const bool narrow = t.bo == 256 && wide_narrow<4>(O);
+        const size_t nbo = narrow ? O / t.bo : cdiv(O, t.bo);
+        const size_t wgs = nbo * cdiv(M, t.bm) * nsplit;
+        const int n = (int)((wgs + cus - 1) / cus);           // the busiest CU's
+        const float last = (float)((wgs - 1) % cus + 1) / cus;  // CUs with that many
+        const float us = (float)(n / 2) * t.two + (float)(n % 2) * t.one - t.fill * (1.0f - last) +
+                         (narrow ? 10.0f : 0.0f);
+        if (!best || us < tbest) {
+            best = &t;
+            tbest = us;
+        }
+    }
+    return best->run(sg, x, (int)M, (int)K, nm, nsplit);
 }
 
 // checks shared by the MFMA entry points: K a multiple of 32 (stages),

@@ -110,6 +110,32 @@ def test_gemm_mfma_tolerance(hip, orc, M, O, K):
     assert nrm <= 2e-3 and same > 0.9
 
 
+# The tile shape follows the call's size; an element's k16 steps are summed
+# in the same order in all of them, so a call of many rows gives bit for bit
+# what 64-row calls (the smallest tile) give. Row and output edges of the
+# 128- to 256-wide tiles, a last output tile of at most 64 outputs and one of
+# more, output counts that are not a multiple of 8 (element stores), K of one
+# stage, of half a stage and with an odd half stage.
+@pytest.mark.parametrize("M,O,K", [(4096, 576, 64), (2300, 4160, 2048), (1025, 12352, 96),
+                                   (700, 12353, 32), (1537, 8200, 160), (769, 12356, 2080),
+                                   (385, 12320, 64), (129, 12352, 192), (3001, 2049, 1056)])
+def test_gemm_mfma_tile_shapes_agree(hip, M, O, K):
+    import torch
+    print(f"[proj] shapes M={M} O={O} K={K}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + O + K)
+    w = (torch.randn(O, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    y = torch.zeros((M, O), dtype=torch.bfloat16, device="cuda")
+    hip.bf16_gemm_dev(w, x, y, exact=False)
+    part = torch.zeros_like(y)
+    for m in range(0, M, 64):
+        hip.bf16_gemm_dev(w, x[m:m + 64], part[m:m + 64], exact=False)
+    assert torch.equal(y.view(torch.int16), part.view(torch.int16))
+    r = x.double() @ w.double().t().contiguous()
+    assert float((y.double() - r).norm() / r.norm()) <= 2e-3      # rnd alone: 1.7e-3
+
+
 def test_gemm_mfma_refuses_unaligned_k(hip):
     """K not a multiple of 32: the MFMA GEMM returns "unsupported" (the
     caller runs the exact kernel or its CPU op), never a wrong result."""
