@@ -66,10 +66,15 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Per-call sequence metadata by value (no upload for small batches).
 constexpr int kPrefillInline = 400;
+constexpr int kScanOrder = 128;
 struct ChunkSeqs {
     int32_t n;
     int32_t cu[kPrefillInline + 1];    // token offsets
     int32_t coff[kPrefillInline + 1];  // chunk offsets
+    // the scan's order of the sequences, longest first (up to kScanOrder of
+    // them, for which the arguments have room: with more, the scan's grid is
+    // many rounds of the chip and its end a small part of it)
+    uint16_t order[kScanOrder];
 };
 
 __device__ __forceinline__ int seq_of(const int32_t *off, int n, int x) {
@@ -674,9 +679,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
 }
 
 // Chunk-to-chunk scan of one 16-column slice of one head's state.
-// Block index = cb * (B*hv) + (s*hv + h): the 8 slices of a head share
-// their operand reads, and with B*hv a multiple of 8 they land on the same
-// XCD (blocks are dealt round-robin over the 8 XCDs) and so share its L2.
+// Block index = (rank * NCB + cb) * hv + h for the rank-th longest sequence:
+// the 8 slices of a head share their operand reads, and with hv a multiple
+// of 8 they land on the same XCD (blocks are dealt round-robin over the 8
+// XCDs) and so share its L2. Longest first: a long sequence's slices walk
+// their chunks one after the other, and started behind the short ones' they
+// ran on alone at the end (lengths 997, 5, 43, 13, 65, 75, slices of a
+// sequence spread over the grid: 75 us; longest first 45).
 // 512 threads in two roles, two wavefronts per SIMD:
 //   waves 0-3 carry the recurrence: D = U - W S0 (rows 16w..), then
 //             S1^T = G_C S0^T + Dp^T K (state rows 32w..);
@@ -754,9 +763,9 @@ __global__ __launch_bounds__(512) void k_gdn_chunk_scan(
     const int32_t *__restrict__ slots) {
     const int hv = hk * REP;
     const size_t vd = (size_t)hv * DV;
-    const int nsh = sq.n * hv;
-    const int cb = blockIdx.x / nsh, sh = blockIdx.x % nsh;
-    const int s = sh / hv, h = sh % hv, kh = h / REP;
+    const int h = blockIdx.x % hv, kh = h / REP, cb = blockIdx.x / hv % NCB;
+    const int rank = blockIdx.x / (hv * NCB);
+    const int s = sq.n <= kScanOrder ? sq.order[rank] : rank;
     const int32_t *cu = dmeta ? dmeta : sq.cu;
     const int32_t *coff = dmeta ? dmeta + sq.n + 1 : sq.coff;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1032,6 +1041,13 @@ static int gdn_prefill_run(const ApusHipGdnLayer *L, size_t B, const int32_t *cu
     }
     ChunkSeqs sq;
     sq.n = (int32_t)B;
+    if (B <= (size_t)kScanOrder) {
+        for (size_t s = 0; s < B; s++) sq.order[s] = (uint16_t)s;
+        std::sort(sq.order, sq.order + B, [&](uint16_t i, uint16_t j) {
+            const int32_t ni = coff[i + 1] - coff[i], nj = coff[j + 1] - coff[j];
+            return ni != nj ? ni > nj : i < j;
+        });
+    }
     const int32_t *dmeta, *kmeta;
     if (B <= (size_t)kPrefillInline) {
         memcpy(sq.cu, cu, (B + 1) * 4);
