@@ -233,9 +233,10 @@ __device__ __forceinline__ void split8(const float (&x)[8], u16x8 &hi, u16x8 &lo
 constexpr int CKP = DK + 8;            // bf16 row stride of the code copies
 
 // Two channels' 4-tap conv sums (tap order, one rounding per mul and add,
-// c/gdn.h:19-33), rounded to bf16 codes by one hardware round-to-nearest-
-// even conversion (v_cvt_pk_bf16_f32): the codes conv_sum4_code gives for
-// finite sums.
+// c/gdn.h:19-33; a product of bf16 values is exact in fp32, so the fused
+// form rounds where they do, products below 2^-126 aside), rounded to bf16
+// codes by one hardware round-to-nearest-even conversion
+// (v_cvt_pk_bf16_f32): the codes conv_sum4_code gives for finite sums.
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t conv_sum4_pair(const float (&w0)[4], const float (&w1)[4],
@@ -243,15 +244,13 @@ __device__ __forceinline__ uint32_t conv_sum4_pair(const float (&w0)[4], const f
                                                    uint32_t x3) {
     auto lo = [](uint32_t v) { return __uint_as_float(v << 16); };
     auto hi = [](uint32_t v) { return __uint_as_float(v & 0xffff0000u); };
-    float a = 0.0f, c = 0.0f;
-    a = a + w0[0] * lo(x0);
-    c = c + w1[0] * hi(x0);
-    a = a + w0[1] * lo(x1);
-    c = c + w1[1] * hi(x1);
-    a = a + w0[2] * lo(x2);
-    c = c + w1[2] * hi(x2);
-    a = a + w0[3] * lo(x3);
-    c = c + w1[3] * hi(x3);
+    float a = fmaf(w0[0], lo(x0), 0.0f), c = fmaf(w1[0], hi(x0), 0.0f);
+    a = fmaf(w0[1], lo(x1), a);
+    c = fmaf(w1[1], hi(x1), c);
+    a = fmaf(w0[2], lo(x2), a);
+    c = fmaf(w1[2], hi(x2), c);
+    a = fmaf(w0[3], lo(x3), a);
+    c = fmaf(w1[3], hi(x3), c);
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, c}, bf16x2_t));
 }
 constexpr int TG = 16;                         // tokens per conv work item
@@ -293,18 +292,40 @@ __device__ __forceinline__ void conv_rows16(const uint16_t *__restrict__ qkv, si
         R.w1[i] = bf2f(conv_w[(gcol + 1) * 4 + i]);
     }
 }
-// conv sums, then the SiLU of each code from the bf16-code table
-// (rnd(co sigmoid(co)) is a function of the code co; the table holds the
-// reference's value for every code). Gathering it costs less than the fp32
-// fast path with its exponential and reciprocal (config 1: WY 95 -> 90 us).
+// conv sums, then the SiLU of each code: channel gcol's from the bf16-code
+// table (it holds the reference's value for every code), channel gcol + 1's
+// by the fp32 formula of silu_fast (gdn_dev.h) and from the table where that
+// formula's rounding is in doubt (about one code in 2000) or the code lies
+// outside [2^-60, 16]. A gather of 64 random codes keeps the address unit
+// busy about as long as the formula keeps the VALU, so one of each per pair
+// runs on both (4096 tokens: WY 81.6 us with every code gathered, 81.9 with
+// every code by the formula, 75.8 so). f1: bit TG - 1 - j: code j in doubt.
 __device__ __forceinline__ void conv_codes16(const ConvRows &R, int tg, int nt,
                                              const uint16_t *__restrict__ silu_bf,
                                              uint16_t (&c0)[TG], uint16_t (&c1)[TG]) {
+    uint32_t cc[TG], f1 = 0;
+    uint32_t amax = 0, amin = 0xffffffffu;
 #pragma unroll
     for (int j = 0; j < TG; j++) {
-        const uint32_t cc = conv_sum4_pair(R.w0, R.w1, R.x[j], R.x[j + 1], R.x[j + 2], R.x[j + 3]);
-        c0[j] = silu_bf[cc & 0xffffu];
-        c1[j] = silu_bf[cc >> 16];
+        cc[j] = conv_sum4_pair(R.w0, R.w1, R.x[j], R.x[j + 1], R.x[j + 2], R.x[j + 3]);
+        c0[j] = silu_bf[cc[j] & 0xffffu];
+    }
+#pragma unroll
+    for (int j = 0; j < TG; j++) {
+        const float x1 = __uint_as_float(cc[j] & 0xffff0000u);
+        constexpr float L2E = 1.44269504088896341f;
+        const float p1 = x1 * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x1 * -L2E));
+        amax = max(amax, cc[j] & 0x7fff0000u);
+        amin = min(amin, cc[j] & 0x7fff0000u);
+        f1 = f1 + f1 + ((__float_as_uint(p1) << 16) + 0x80100000u < 0x210000u ? 1u : 0u);
+        const __bf16 h = (__bf16)p1;
+        c1[j] = __builtin_bit_cast(uint16_t, h);
+    }
+    if (!(amax <= 0x41800000u && amin >= 0x21800000u)) f1 = 0xffffu;
+    if (__builtin_amdgcn_ballot_w64(f1 != 0)) {
+#pragma unroll
+        for (int j = 0; j < TG; j++)
+            if (f1 >> (TG - 1 - j) & 1u) c1[j] = silu_bf[cc[j] >> 16];
     }
 #pragma unroll
     for (int j = 0; j < TG; j++)

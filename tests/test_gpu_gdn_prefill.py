@@ -82,6 +82,44 @@ def test_prefill_strong_decay(hip, orc):
                  a_scale=2.0, tag="strong_decay")
 
 
+def test_prefill_silu_every_code(hip, orc):
+    """The chunk kernel's SiLU (from the table for one channel of a pair, by
+    formula with the table behind it for the other) on every bf16 code of
+    magnitude 2^-80 .. 2^40 above -64 (below it the product goes to 0): 16 one-token sequences from a zero state, whose
+    conv passes the codes through (last tap 1). S = beta k v^T then, so
+    column j shows v_j = SiLU(code) to the chunk form's own 1e-5, against
+    2^-8 for a code that is one ulp off."""
+    import torch
+    dims = synth.GDN_DIMS
+    hk, hv, dk, dv = dims
+    rng = np.random.default_rng(8)
+    B, cd, kd = 16, 2 * hk * dk + hv * dv, hk * dk
+    w = synth.gdn_weights(rng)
+    w["conv_w"] = np.zeros((cd, 4), np.uint16)
+    w["conv_w"][:, 3] = 0x3F80
+    tok = synth.gdn_tokens(rng, B)
+    codes = rng.permutation(np.arange(1 << 16, dtype=np.uint32)).astype(np.uint16)
+    exp = (codes >> 7) & 0xFF
+    codes = np.where((exp >= 127 - 80) & (exp <= np.where(codes >> 15, 127 + 5, 127 + 40)), codes,
+                     0x3F80)
+    tok["qkv"][:, 2 * kd:] = codes.reshape(B, hv * dv)
+    conv, S = synth.gdn_state(rng, B, zero=True)
+    cu = np.arange(B + 1, dtype=np.int32)
+    S_o = S.copy()
+    orc.gdn_mixer(dims, w, cu, tok["qkv"], tok["z"], tok["a"], tok["b"], conv.copy(), S_o)
+    layer = hip.gdn_layer(dims, {k: _dev(torch, v) for k, v in w.items()})
+    t = {k: _dev(torch, v) for k, v in tok.items()}
+    dS = torch.zeros((B, hv, dk, dv), device="cuda")
+    out = torch.empty_like(dS)
+    y = torch.empty((B, hv * dv), dtype=torch.int16, device="cuda")
+    hip.gdn_prefill(layer, cu, t["qkv"], t["z"], t["a"], t["b"], _dev(torch, conv), dS, y)
+    hip.gdn_state_unpack(dS, out)
+    torch.cuda.synchronize()
+    r = S_o.astype(np.float64)
+    err = np.abs(out.cpu().numpy() - r).max(axis=2) / np.abs(r).max(axis=2)
+    assert err.max() <= 1e-4, float(err.max())
+
+
 def test_prefill_then_decode(hip, orc):
     """Prefill a prompt then decode one token from the device state: the
     state layout and conv state the prefill leaves are what decode reads."""
