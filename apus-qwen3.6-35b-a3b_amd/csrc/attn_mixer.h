@@ -44,16 +44,20 @@ __device__ __forceinline__ size_t kv_block_id_u(const KvRef &r, int h, int b) {
 // ---- per-call sequence metadata ------------------------------------------
 // Passed by value as a kernel argument for up to kAttnInlineSeqs sequences
 // (no host->device copy on the decode path), else as a device array
-// cu[B+1] | pos0[B] | ccap[B+1] | hd[B].
-constexpr int kAttnInlineSeqs = 224;
-struct AttnSeqs {
+// cu[B+1] | pos0[B] | ccap[B+1] | hd[B]. Calls of up to kAttnFewSeqs
+// sequences pass a short form: a launch copies its whole argument block, and
+// the kernel reads it from the host (attn_decode_kv's four launches at one
+// sequence: 1.5 us less).
+constexpr int kAttnInlineSeqs = 224, kAttnFewSeqs = 8;
+template <int N> struct AttnSeqsN {
     int32_t n;                          // sequences
     int32_t T1, T2;                     // keys per score / P.V wavefront (multiples of 64)
-    int32_t cu[kAttnInlineSeqs + 1];    // token offsets
-    int32_t pos0[kAttnInlineSeqs];      // tokens already cached
-    int32_t ccap[kAttnInlineSeqs + 1];  // prefix sums of cap = ceil64(pos0 + tokens)
-    int32_t hd[kAttnInlineSeqs];        // block-table row of each sequence
+    int32_t cu[N + 1];                  // token offsets
+    int32_t pos0[N];                    // tokens already cached
+    int32_t ccap[N + 1];                // prefix sums of cap = ceil64(pos0 + tokens)
+    int32_t hd[N];                      // block-table row of each sequence
 };
+using AttnSeqs = AttnSeqsN<kAttnInlineSeqs>;
 
 int attn_check_layer(const ApusHipAttnLayer *L);
 

@@ -18,7 +18,8 @@
 //   k_attn_prep     q/k (1+w) RMSNorm, RoPE, K append; V append (other
 //                   blocks of the same launch)
 //   k_attn_scores   A = rnd(rnd(q.k)*scale) on MFMA 16x16x32 bf16 into a
-//                   bf16 score buffer, per-segment (max, sum exp)
+//                   bf16 score buffer, per-segment (max, sum exp);
+//                   k_attn_scores_few for calls of few keys
 //   k_attn_pv       P = rnd(exp(A-m)/s) with the pair's global (m, s) --
 //                   the reference's normalised bf16 probabilities
 //                   (c/attn.h:354-360) -- times V on MFMA, fp32 partials
@@ -31,6 +32,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/apus_hip.h"
@@ -84,7 +86,8 @@ __host__ __device__ inline int seq_of(const int32_t *off, int n, int x) {
 struct Meta {
     const int32_t *cu, *pos0, *ccap, *hd;
 };
-__device__ __forceinline__ Meta meta_of(const AttnSeqs &sq, const int32_t *dmeta) {
+template <int N>
+__device__ __forceinline__ Meta meta_of(const AttnSeqsN<N> &sq, const int32_t *dmeta) {
     if (!dmeta) return Meta{sq.cu, sq.pos0, sq.ccap, sq.hd};
     const int n = sq.n;
     return Meta{dmeta, dmeta + n + 1, dmeta + 2 * n + 1, dmeta + 3 * n + 2};
@@ -115,7 +118,7 @@ constexpr int kVappLds = 32 * PRS * 2;       // the V append block's staged rows
 constexpr int kPrepKernLds = sizeof(PrepLds) > kVappLds ? sizeof(PrepLds) : kVappLds;
 
 __device__ __forceinline__ void prep_block(
-    int bid, PrepLds &L, const Meta &mt, const AttnSeqs &sq, const uint16_t *__restrict__ qg,
+    int bid, PrepLds &L, const Meta &mt, int nseq, const uint16_t *__restrict__ qg,
     const uint16_t *__restrict__ kin, const uint16_t *__restrict__ qn_w,
     const uint16_t *__restrict__ kn_w, const uint16_t *__restrict__ rope, const KvRef &kv,
     uint16_t *__restrict__ qn, int nh, int nkv, int nrows, int rpb, uint16_t *__restrict__ tr_kf,
@@ -136,7 +139,7 @@ __device__ __forceinline__ void prep_block(
     // no wait drains the stream.
     const int tt0 = r0 / nslot, ntk = (r0 + nr - 1) / nslot - tt0 + 1;
     if (tid < ntk) {
-        const int tt = tt0 + tid, s = seq_of(cu, sq.n, tt);
+        const int tt = tt0 + tid, s = seq_of(cu, nseq, tt);
         tpos[tid] = pos0[s] + (tt - cu[s]);
         thd[tid] = mt.hd[s];
     }
@@ -286,8 +289,9 @@ __device__ __forceinline__ void vappend_block(int bid, uint16_t *vt, const Meta 
 // One launch for both: blocks [0, nprep) are prep blocks of rpb rows,
 // the rest V append blocks (B * nkv * maxnb of them). Neither reads what
 // the other writes (the K and V caches, qn), so they need no order.
+template <int N>
 __global__ __launch_bounds__(256) void k_attn_prep(
-    AttnSeqs sq, const int32_t *__restrict__ dmeta, const uint16_t *__restrict__ qg,
+    AttnSeqsN<N> sq, const int32_t *__restrict__ dmeta, const uint16_t *__restrict__ qg,
     const uint16_t *__restrict__ kin, const uint16_t *__restrict__ vin,
     const uint16_t *__restrict__ qn_w, const uint16_t *__restrict__ kn_w,
     const uint16_t *__restrict__ rope, KvRef kv, uint16_t *__restrict__ qn, int nh, int nkv,
@@ -295,7 +299,7 @@ __global__ __launch_bounds__(256) void k_attn_prep(
     __shared__ __attribute__((aligned(16))) char lds[kPrepKernLds];
     const Meta mt = meta_of(sq, dmeta);
     if ((int)blockIdx.x < nprep)
-        prep_block((int)blockIdx.x, *reinterpret_cast<PrepLds *>(lds), mt, sq, qg, kin, qn_w,
+        prep_block((int)blockIdx.x, *reinterpret_cast<PrepLds *>(lds), mt, sq.n, qg, kin, qn_w,
                    kn_w, rope, kv, qn, nh, nkv, nrows, rpb, tr_kf, qrows);
     else
         vappend_block((int)blockIdx.x - nprep, reinterpret_cast<uint16_t *>(lds), mt, vin, kv,
@@ -447,6 +451,13 @@ __device__ __forceinline__ const uint16_t *uniform_ptr(const uint16_t *p) {
 __device__ __forceinline__ const uint16_t *kblock(const KvRef &kv, int hd, const Seg &g, int nkv,
                                                   int b) {
     return uniform_ptr(kv.k + (kv_block_id_u(kv, hd, b) * nkv + g.kvh) * KVB * D);
+}
+
+// (m, s) of two sets of scores joined: the max and the sum of e^{A - max}
+__device__ __forceinline__ void stat_join(float &m, float &s, float mo, float so) {
+    const float mm = fmaxf(m, mo);
+    s = mm > -INFINITY ? s * exp_fast(m - mm) + so * exp_fast(mo - mm) : 0.0f;
+    m = mm;
 }
 
 // The streaming wavefront's part for one segment whose sequence has NR
@@ -658,9 +669,7 @@ __device__ __forceinline__ void scores_seg(const Meta &mt, const Seg &c,
 #pragma unroll
         for (int off = 16; off < 64; off <<= 1) {
             const float mo = __shfl_xor(m, off), lo = __shfl_xor(ls, off);
-            const float mm = fmaxf(m, mo);
-            ls = mm > -INFINITY ? ls * exp_fast(m - mm) + lo * exp_fast(mo - mm) : 0.0f;
-            m = mm;
+            stat_join(m, ls, mo, lo);
         }
         if (q4 == 0 && vrow[rb]) stats[(size_t)c.slot * kRows + rb * 16 + c16] = make_float2(m, ls);
     }
@@ -767,6 +776,136 @@ __global__ __launch_bounds__(64 * (ScoresShape<NRB>::W + 1)) void k_attn_scores(
     }
 }
 
+// ---- k_attn_scores_few: the scores of a call of up to kFewKeys keys ------
+// One workgroup of 4 wavefronts per run: wavefront j takes keys 16 j .. +15
+// of each 64-key group, stores its scores itself (8 bytes a lane) and the
+// workgroup folds the four (max, sum) of a row in LDS. k_attn_scores keeps
+// 7 to 11 runs on a CU and passes the scores of each run through one more
+// wavefront, which pays when every CU streams for long; with few keys it
+// leaves most CUs idle and a group is a chain of four loads (one sequence at
+// 1500 positions: 14.0 us, here 5.4).
+template <int NR>
+__device__ __forceinline__ void scores_few_seg(const Meta &mt, const Seg &c,
+                                               const uint16_t *__restrict__ qn, const KvRef &kv,
+                                               int nh, int nkv, float scale,
+                                               uint16_t *__restrict__ As,
+                                               float2 *__restrict__ stats, uint4 *stg,
+                                               float2 (*fold)[kRows]) {
+    const int l = threadIdx.x & 63, c16 = l & 15, q4 = l >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int hd = __builtin_amdgcn_readfirstlane(mt.hd[c.s]);
+    const int blast = (c.k1 - 1) >> 5;
+    // rows g0 + 16 wave + 0 .. 15 (one cache block), two whole rows a load;
+    // rows past the segment's end re-read its last one (never stored)
+    u16x8 f[D / 32];
+    auto load_k = [&](int g0) {
+        const int kb = g0 + 16 * wave;
+        const uint16_t *blk = kblock(kv, hd, c, nkv, min(kb >> 5, blast));
+#pragma unroll
+        for (int i = 0; i < D / 32; i++) {
+            const int key = min(kb + 2 * i + (l >> 5), c.k1 - 1);
+            f[i] = __builtin_nontemporal_load((gu16x8p)(blk + (size_t)(key & 31) * D + (l & 31) * 8));
+        }
+    };
+    load_k(c.k0);
+    bf16x8 qf[NR][D / 32];
+    int lim[NR];
+    bool vrow[NR];
+    float mrun[NR], lrun[NR];
+#pragma unroll
+    for (int rb = 0; rb < NR; rb++) {
+        const int n = rb * 16 + c16, t = n / GRP;
+        vrow[rb] = t < c.tq;
+        lim[rb] = c.pos0 + t;
+        mrun[rb] = -INFINITY;
+        lrun[rb] = 0.0f;
+        const uint16_t *qrow =
+            qn + ((size_t)(mt.cu[c.s] + (vrow[rb] ? t : 0)) * nh + c.kvh * GRP + n % GRP) * D;
+#pragma unroll
+        for (int ds = 0; ds < D / 32; ds++) {
+            const bf16x8 v = ld_bf16x8(qrow + ds * 32 + q4 * 8);
+            qf[rb][ds] = vrow[rb] ? v : bf16x8{};
+        }
+    }
+    for (int g0 = c.k0; g0 < c.k1; g0 += 64) {
+#pragma unroll
+        for (int i = 0; i < D / 32; i++)
+            stg[(2 * i + (l >> 5)) * 33 + (l & 31)] = __builtin_bit_cast(uint4, f[i]);
+        if (g0 + 64 < c.k1) load_k(g0 + 64);
+        f32x4 acc[NR];
+#pragma unroll
+        for (int rb = 0; rb < NR; rb++) acc[rb] = f32x4{};
+#pragma unroll
+        for (int ds = 0; ds < D / 32; ds++) {
+            const bf16x8 k = __builtin_bit_cast(bf16x8, stg[c16 * 33 + ds * 4 + q4]);
+#pragma unroll
+            for (int rb = 0; rb < NR; rb++)
+                acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k, qf[rb][ds], acc[rb], 0, 0, 0);
+        }
+        // this lane: keys kq .. kq + 3 of row rb * 16 + c16
+        const int kq = g0 + 16 * wave + 4 * q4;
+#pragma unroll
+        for (int rb = 0; rb < NR; rb++) {
+            if (!vrow[rb] || kq >= c.k1) continue;
+            const uint32_t s0 = pack2(acc[rb][0] * scale, acc[rb][1] * scale);
+            const uint32_t s1 = pack2(acc[rb][2] * scale, acc[rb][3] * scale);
+            *reinterpret_cast<uint2 *>(As + c.abase + a_index(rb * 16 + c16, kq, c.cap)) = make_uint2(s0, s1);
+            const float a[4] = {__uint_as_float(s0 << 16), __uint_as_float(s0 & 0xffff0000u),
+                                __uint_as_float(s1 << 16), __uint_as_float(s1 & 0xffff0000u)};
+            const int last = min(lim[rb], c.k1 - 1) - kq;      // the last key that counts
+            float mn = mrun[rb];
+#pragma unroll
+            for (int e = 0; e < 4; e++) mn = fmaxf(mn, e <= last ? a[e] : -INFINITY);
+            if (mn == -INFINITY) continue;
+            float add = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (e <= last) add += __builtin_amdgcn_exp2f(fmaf(a[e], kL2E, -mn * kL2E));
+            lrun[rb] = lrun[rb] * __builtin_amdgcn_exp2f((mrun[rb] - mn) * kL2E) + add;
+            mrun[rb] = mn;
+        }
+    }
+    __syncthreads();                           // fold's readers of the segment before
+#pragma unroll
+    for (int rb = 0; rb < NR; rb++) {
+#pragma unroll
+        for (int off = 16; off < 64; off <<= 1) {
+            const float mo = __shfl_xor(mrun[rb], off), so = __shfl_xor(lrun[rb], off);
+            stat_join(mrun[rb], lrun[rb], mo, so);
+        }
+        if (q4 == 0) fold[wave][rb * 16 + c16] = make_float2(mrun[rb], lrun[rb]);
+    }
+    __syncthreads();
+    if (threadIdx.x < NR * 16 && (int)threadIdx.x / GRP < c.tq) {
+        float2 r = fold[0][threadIdx.x];
+#pragma unroll
+        for (int j = 1; j < 4; j++) stat_join(r.x, r.y, fold[j][threadIdx.x].x, fold[j][threadIdx.x].y);
+        stats[(size_t)c.slot * kRows + threadIdx.x] = r;
+    }
+}
+
+template <int NRB, int N>
+__global__ __launch_bounds__(256) void k_attn_scores_few(
+    AttnSeqsN<N> sq, const int32_t *__restrict__ dmeta, const uint16_t *__restrict__ qn, KvRef kv,
+    int nh, int nkv, float scale, uint16_t *__restrict__ As, float2 *__restrict__ stats) {
+    __shared__ uint4 stg[4][16 * 33];
+    __shared__ float2 fold[4][kRows];
+    const Meta mt = meta_of(sq, dmeta);
+    const int n = sq.n, T = sq.T1, total = nkv * mt.ccap[n], run = (int)blockIdx.x;
+    const int x1 = min(run * T + T, total);
+    for (int x = run * T; x < x1;) {
+        Seg g;
+        int xn;
+        if (seg_at(mt, n, nkv, run, x, x1, g, &xn)) {
+            if (NRB == 2 && g.tq <= 2)
+                scores_few_seg<1>(mt, g, qn, kv, nh, nkv, scale, As, stats, stg[threadIdx.x >> 6], fold);
+            else
+                scores_few_seg<NRB>(mt, g, qn, kv, nh, nkv, scale, As, stats, stg[threadIdx.x >> 6], fold);
+        }
+        x = xn;
+    }
+}
+
 // ---- k_attn_pv: one run of T2 keys per item ------------------------------
 // O^T[d][row] = sum_key V^T[d][key] P^T[key][row] on MFMA 16x16x32: the
 // transposed V blocks are the A operand (4 lanes read 64 contiguous bytes
@@ -777,14 +916,14 @@ __global__ __launch_bounds__(64 * (ScoresShape<NRB>::W + 1)) void k_attn_scores(
 // P.V over one segment for a sequence with NR row blocks of queries; this
 // wavefront owns d blocks hb*NB .. +NB
 template <int NR, int NB>
-__device__ __forceinline__ void pv_seg(const Meta &mt, const Seg &c, int hb, const AttnSeqs &sq,
+__device__ __forceinline__ void pv_seg(const Meta &mt, const Seg &c, int hb, int T1,
                                        const KvRef &kv, int nkv, const uint16_t *__restrict__ As,
                                        const float2 *__restrict__ stats, float *__restrict__ Op) {
     const int l = threadIdx.x, c16 = l & 15, q4 = l >> 4;
 
     // global (max, sum) of each row over the pair's score segments
     int w0, w1;
-    pair_runs(mt, nkv, c.s, c.kvh, sq.T1, &w0, &w1);
+    pair_runs(mt, nkv, c.s, c.kvh, T1, &w0, &w1);
     const int p = c.s * nkv + c.kvh;
     float m[NR], rsum[NR];
     bool vrow[NR];
@@ -796,23 +935,24 @@ __device__ __forceinline__ void pv_seg(const Meta &mt, const Seg &c, int hb, con
         lim[rb] = c.pos0 + t;
         float mm = -INFINITY, ss = 0.0f;
         if (vrow[rb]) {
-            // eight segments' statistics in flight at a time (a long pair
-            // has dozens; one dependent load each would serialise their
-            // latencies)
-            for (int w = w0; w <= w1; w += 8) {
+            // every fourth segment's statistics (the lanes q4 = 0..3 of a row
+            // take one residue each), eight in flight at a time: a pair of a
+            // long context has hundreds, and one lane reading them all made
+            // P.V of one sequence at 32,000 positions 60 us
+            for (int w = w0 + q4; w <= w1; w += 32) {
                 float2 st[8];
 #pragma unroll
                 for (int i = 0; i < 8; i++)
-                    st[i] = w + i <= w1 ? stats[(size_t)(p + w + i) * kRows + n]
-                                        : make_float2(-INFINITY, 0.0f);
+                    st[i] = w + 4 * i <= w1 ? stats[(size_t)(p + w + 4 * i) * kRows + n]
+                                            : make_float2(-INFINITY, 0.0f);
 #pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    if (st[i].x == -INFINITY) continue;
-                    const float mn = fmaxf(mm, st[i].x);
-                    ss = ss * exp_fast(mm - mn) + st[i].y * exp_fast(st[i].x - mn);
-                    mm = mn;
-                }
+                for (int i = 0; i < 8; i++) stat_join(mm, ss, st[i].x, st[i].y);
             }
+        }
+#pragma unroll
+        for (int off = 16; off < 64; off <<= 1) {
+            const float mo = __shfl_xor(mm, off), so = __shfl_xor(ss, off);
+            stat_join(mm, ss, mo, so);
         }
         // P = rnd(e^{A - m} / s) formed as rnd(exp2(A log2(e) - K)), K =
         // m log2(e) + log2(s): the division folded into the exponent (a
@@ -903,9 +1043,9 @@ __device__ __forceinline__ void pv_seg(const Meta &mt, const Seg &c, int hb, con
     }
 }
 
-template <int NRB, int DH>
+template <int NRB, int DH, int N>
 __global__ __launch_bounds__(64) void k_attn_pv(
-    AttnSeqs sq, const int32_t *__restrict__ dmeta, KvRef kv, int nkv,
+    AttnSeqsN<N> sq, const int32_t *__restrict__ dmeta, KvRef kv, int nkv,
     const uint16_t *__restrict__ As, const float2 *__restrict__ stats, float *__restrict__ Op) {
     const Meta mt = meta_of(sq, dmeta);
     constexpr int NB = D / 16 / DH;            // 16-row d blocks of this wavefront
@@ -919,46 +1059,61 @@ __global__ __launch_bounds__(64) void k_attn_pv(
         if (seg_at(mt, n, nkv, run, x, x1, g, &xn)) {
             // a sequence with at most 2 tokens fills one row block
             if (NRB == 2 && g.tq <= 2)
-                pv_seg<1, NB>(mt, g, hb, sq, kv, nkv, As, stats, Op);
+                pv_seg<1, NB>(mt, g, hb, sq.T1, kv, nkv, As, stats, Op);
             else
-                pv_seg<NRB, NB>(mt, g, hb, sq, kv, nkv, As, stats, Op);
+                pv_seg<NRB, NB>(mt, g, hb, sq.T1, kv, nkv, As, stats, Op);
         }
         x = xn;
     }
 }
 
-// ---- k_attn_combine: one block per (token, kv head, 4 of its q heads) --
+// ---- k_attn_combine: one block per (token, kv head, 4 / SP of its q heads)
 // A thread owns 4 consecutive d of one (token, q head) row: its gate codes
 // are loaded first, then up to 16 of the pair's run partials at once
 // (float4 each), summed in run order from 0.0f; rnd, times
 // rnd(sigmoid(gate)). One block per (token, q head) with a thread per d
 // needed three rounds of resident waves on config 4, each a chain of
-// dependent loads.
+// dependent loads. SP = 4 wavefronts share a row of a pair of many runs,
+// each summing a quarter of them, the quarters then summed in order (one
+// sequence at 32,000 positions, 500 runs a pair: 37 us with SP = 1, 12 with
+// 4).
+template <int SP, int N>
 __global__ __launch_bounds__(256) void k_attn_combine(
-    AttnSeqs sq, const int32_t *__restrict__ dmeta, const float *__restrict__ Op,
+    AttnSeqsN<N> sq, const int32_t *__restrict__ dmeta, const float *__restrict__ Op,
     const uint16_t *__restrict__ qg, int nh, int nkv, uint16_t *__restrict__ y,
     const uint16_t *__restrict__ sig_bf, uint16_t *__restrict__ tr_attno) {
     const Meta mt = meta_of(sq, dmeta);
-    const int half = blockIdx.x & 1, tk = blockIdx.x >> 1;
+    constexpr int HB = 4 / SP, NBH = GRP / HB;      // q heads of a block, blocks of a kv head
+    const int part = blockIdx.x % NBH, tk = blockIdx.x / NBH;
     const int tt = tk / nkv, kvh = tk % nkv;
     const int s = seq_of(mt.cu, sq.n, tt), t = tt - mt.cu[s];
-    const int g = half * (GRP / 2) + (threadIdx.x >> 6), h = kvh * GRP + g, n = t * GRP + g;
+    const int wave = threadIdx.x >> 6, quarter = wave % SP;
+    const int g = part * HB + wave / SP, h = kvh * GRP + g, n = t * GRP + g;
     const int d = (threadIdx.x & 63) * 4;
     const size_t row = (size_t)tt * nh + h;
     const uint2 gc = *reinterpret_cast<const uint2 *>(qg + row * 2 * D + D + d);
     int w0, w1;
     pair_runs(mt, nkv, s, kvh, sq.T2, &w0, &w1);
-    const int nw = w1 - w0;
+    const int share = (w1 - w0) / SP + 1, first = quarter * share;
+    const int last = min(w1 - w0, first + share - 1);
     const float *P0 = Op + ((size_t)(s * nkv + kvh + w0) * kRows + n) * D + d;
     f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int w = 0; w <= nw; w += 16) {
+    for (int w = first; w <= last; w += 16) {
         f32x4 v[16];
 #pragma unroll
         for (int i = 0; i < 16; i++)
-            v[i] = *reinterpret_cast<const f32x4 *>(P0 + (size_t)min(w + i, nw) * kRows * D);
+            v[i] = *reinterpret_cast<const f32x4 *>(P0 + (size_t)min(w + i, last) * kRows * D);
 #pragma unroll
         for (int i = 0; i < 16; i++)
-            if (w + i <= nw) sum += v[i];
+            if (w + i <= last) sum += v[i];
+    }
+    if (SP > 1) {
+        __shared__ f32x4 parts[4][64];
+        parts[wave][threadIdx.x & 63] = sum;
+        __syncthreads();
+        if (quarter) return;
+#pragma unroll
+        for (int q = 1; q < SP; q++) sum += parts[wave + q][threadIdx.x & 63];
     }
     const uint16_t code[4] = {(uint16_t)gc.x, (uint16_t)(gc.x >> 16), (uint16_t)gc.y,
                               (uint16_t)(gc.y >> 16)};
@@ -1028,15 +1183,30 @@ KvRef kv_flat(uint16_t *kcache, uint16_t *vcache, size_t max_seq) {
     return KvRef{kcache, vcache, nullptr, (int32_t)(max_seq / KVB)};
 }
 
+// runs of a pair past which four wavefronts sum a row's partials: more than
+// two rounds of the 16 loads that one has in flight
+static const size_t kWidePair = 32;
+
 static size_t ceil64(size_t x) { return (x + 63) / 64 * 64; }
 
-// decode: balanced runs of T keys per wavefront over `total` padded keys,
-// each kernel's grid one round of resident wavefronts (scores: W streaming
-// wavefronts per CU; P.V: two wavefronts per run, each owning half of d,
-// at three wavefronts per SIMD for one row block, two for two)
+// padded keys up to which k_attn_scores_few forms the scores (measured, us a
+// decode call with it / with the ring kernel, one new token: 16 sequences
+// at 2000 positions 35 / 52, 16 at 8000 71 / 81, 64 at 3000 104 / 114; four:
+// 43 / 51, 81 / 90, 120 / 122; 64 at 9000 248 / 245)
+constexpr size_t kFewKeys = (size_t)8192 * 64;
+
+// decode: balanced runs of T keys over `total` padded keys. Scores: one run
+// per streaming wavefront of one round of resident workgroups, or two per CU
+// for k_attn_scores_few (every run costs P.V a statistic: one sequence at
+// 60,000 positions 57 us with two, 92 with eleven). P.V: three runs per CU
+// of two wavefronts each, two while that leaves runs of 256 keys or less (each
+// run writes 8 KiB of partials per row block, so more runs cost more than
+// the wavefronts they add: 64 sequences at 32768 positions, P.V 351 us with
+// three runs per CU, 368 with six).
 static void attn_split_sizes(size_t total, size_t max_tok, size_t cus, int32_t *T1, int32_t *T2) {
-    const size_t w1 = (max_tok <= 2 ? scores_waves_per_block<1>() : scores_waves_per_block<2>()) * cus;
-    const size_t w2 = (max_tok <= 2 ? 3 : 2) * 4 * cus / 2;
+    const size_t ring = max_tok <= 2 ? scores_waves_per_block<1>() : scores_waves_per_block<2>();
+    const size_t w1 = (total <= kFewKeys ? 2 : ring) * cus;
+    const size_t w2 = (total <= 2 * 256 * cus * 3 / 2 ? 2 : 3) * cus;
     *T1 = (int32_t)std::max<size_t>(64, ceil64((total + w1 - 1) / w1));
     *T2 = (int32_t)std::max<size_t>(64, ceil64((total + w2 - 1) / w2));
 }
@@ -1084,6 +1254,19 @@ int attn_meta(size_t B, const int32_t *cu, const int32_t *pos0, const int32_t *r
     return kOk;
 }
 
+// the short form of the metadata of at most kAttnFewSeqs sequences
+static AttnSeqsN<kAttnFewSeqs> few_seqs(const AttnSeqs &s) {
+    AttnSeqsN<kAttnFewSeqs> m;
+    m.n = s.n;
+    m.T1 = s.T1;
+    m.T2 = s.T2;
+    memcpy(m.cu, s.cu, sizeof m.cu);
+    memcpy(m.pos0, s.pos0, sizeof m.pos0);
+    memcpy(m.ccap, s.ccap, sizeof m.ccap);
+    memcpy(m.hd, s.hd, sizeof m.hd);
+    return m;
+}
+
 int attn_prep(const ApusHipAttnLayer *L, const AttnSeqs &sq, const int32_t *dmeta,
               size_t Ttot, size_t max_pos, int maxnb, const uint16_t *qg, const uint16_t *k,
               const uint16_t *v, const KvRef &kv, uint16_t *qn, bool qrows) {
@@ -1093,11 +1276,16 @@ int attn_prep(const ApusHipAttnLayer *L, const AttnSeqs &sq, const int32_t *dmet
     // few rows (decode): small blocks, so they spread over the chip
     const int rpb = nrows < (size_t)8 * PRB * cu_count() ? 8 : PRB;
     const unsigned nprep = cdiv(nrows, rpb), nvapp = (unsigned)(sq.n * L->nkv * maxnb);
-    APUS_TIMED("k_attn_prep",
-               k_attn_prep<<<nprep + nvapp, 256, 0, stream()>>>(
-        sq, dmeta, qg, k, v, L->qn_w, L->kn_w, rope, kv, qn, (int)L->nh, (int)L->nkv,
-        (int)nrows, rpb, (int)nprep, maxnb, attn_trace() ? attn_trace()->kf : nullptr,
-        qrows ? 1 : 0));
+    auto launch = [&](const auto &m) {
+        constexpr int N = sizeof(m.pos0) / 4;
+        APUS_TIMED("k_attn_prep",
+                   k_attn_prep<N><<<nprep + nvapp, 256, 0, stream()>>>(
+                       m, dmeta, qg, k, v, L->qn_w, L->kn_w, rope, kv, qn, (int)L->nh, (int)L->nkv,
+                       (int)nrows, rpb, (int)nprep, maxnb, attn_trace() ? attn_trace()->kf : nullptr,
+                       qrows ? 1 : 0));
+    };
+    if (sq.n <= kAttnFewSeqs) launch(few_seqs(sq));
+    else launch(sq);
     if (int r = launch_check("k_attn_prep")) return r;
     if (const ApusHipAttnTrace *tr = attn_trace()) {
         if (tr->qf && qrows)
@@ -1142,6 +1330,7 @@ int attn_decode_kv(const ApusHipAttnLayer *L, size_t B, const int32_t *cu, const
         max_pos = std::max(max_pos, (size_t)pos0[s] + (size_t)(cu[s + 1] - cu[s]));
         keys += ceil64((size_t)pos0[s] + (size_t)(cu[s + 1] - cu[s]));
     }
+    const size_t max_cap = ceil64(max_pos);
     const size_t total = nkv * keys;
     const size_t nruns1 = (total + sq.T1 - 1) / sq.T1, nruns2 = (total + sq.T2 - 1) / sq.T2;
     uint16_t *qn = (uint16_t *)scratch(kScratchAttnQ, Ttot * L->nh * D * 2);
@@ -1156,35 +1345,40 @@ int attn_decode_kv(const ApusHipAttnLayer *L, size_t B, const int32_t *cu, const
     const ActTables *tabs = act_tables();
     if (!tabs) return kErrHip;
     // one 16-row block covers up to 2 new tokens per sequence (8 heads each)
-    if (mt <= 2) {
-        APUS_TIMED("k_attn_scores",
-                   k_attn_scores<1><<<cdiv(nruns1, scores_waves_per_block<1>()),
-                                      64 * (scores_waves_per_block<1>() + 1), 0, stream()>>>(
-                       sq, dmeta, qn, kv, (int)L->nh, (int)nkv, scale, As, st, (int)nruns1,
-                       spin_limit(), fault_word()));
+    auto launch = [&](auto nrb, const auto &m) {
+        constexpr int NRB = decltype(nrb)::value, N = sizeof(m.pos0) / 4;
+        if (total <= kFewKeys) {
+            APUS_TIMED("k_attn_scores",
+                       k_attn_scores_few<NRB, N><<<(unsigned)nruns1, 256, 0, stream()>>>(
+                           m, dmeta, qn, kv, (int)L->nh, (int)nkv, scale, As, st));
+        } else {
+            APUS_TIMED("k_attn_scores",
+                       k_attn_scores<NRB><<<cdiv(nruns1, scores_waves_per_block<NRB>()),
+                                            64 * (scores_waves_per_block<NRB>() + 1), 0, stream()>>>(
+                           sq, dmeta, qn, kv, (int)L->nh, (int)nkv, scale, As, st, (int)nruns1,
+                           spin_limit(), fault_word()));
+        }
         APUS_LAUNCHED("k_attn_scores");
         APUS_TIMED("k_attn_pv",
-                   k_attn_pv<1, 2><<<(unsigned)(2 * nruns2), 64, 0, stream()>>>(
-                       sq, dmeta, kv, (int)nkv, As, st, Op));
+                   k_attn_pv<NRB, 2, N><<<(unsigned)(2 * nruns2), 64, 0, stream()>>>(
+                       m, dmeta, kv, (int)nkv, As, st, Op));
         APUS_LAUNCHED("k_attn_pv");
-    } else {
-        APUS_TIMED("k_attn_scores",
-                   k_attn_scores<2><<<cdiv(nruns1, scores_waves_per_block<2>()),
-                                      64 * (scores_waves_per_block<2>() + 1), 0, stream()>>>(
-                       sq, dmeta, qn, kv, (int)L->nh, (int)nkv, scale, As, st, (int)nruns1,
-                       spin_limit(), fault_word()));
-        APUS_LAUNCHED("k_attn_scores");
-        APUS_TIMED("k_attn_pv",
-                   k_attn_pv<2, 2><<<(unsigned)(2 * nruns2), 64, 0, stream()>>>(
-                       sq, dmeta, kv, (int)nkv, As, st, Op));
-        APUS_LAUNCHED("k_attn_pv");
-    }
-    APUS_TIMED("k_attn_combine",
-               k_attn_combine<<<(unsigned)(Ttot * nkv * 2), 256, 0, stream()>>>(
-                   sq, dmeta, Op, qg, (int)L->nh, (int)nkv, y, tabs->sig_bf,
-                   attn_trace() ? attn_trace()->attno : nullptr));
-    APUS_LAUNCHED("k_attn_combine");
-    return kOk;
+        auto combine = [&](auto sp) {
+            constexpr int SP = decltype(sp)::value;
+            APUS_TIMED("k_attn_combine",
+                       k_attn_combine<SP, N><<<(unsigned)(Ttot * nkv * 2 * SP), 256, 0, stream()>>>(
+                           m, dmeta, Op, qg, (int)L->nh, (int)nkv, y, tabs->sig_bf,
+                           attn_trace() ? attn_trace()->attno : nullptr));
+        };
+        if (max_cap / sq.T2 > kWidePair) combine(std::integral_constant<int, 4>{});
+        else combine(std::integral_constant<int, 1>{});
+        APUS_LAUNCHED("k_attn_combine");
+        return (int)kOk;
+    };
+    const std::integral_constant<int, 1> one;
+    const std::integral_constant<int, 2> two;
+    if (B <= (size_t)kAttnFewSeqs) return mt <= 2 ? launch(one, few_seqs(sq)) : launch(two, few_seqs(sq));
+    return mt <= 2 ? launch(one, sq) : launch(two, sq);
 }
 
 int kv_paged_ref(const ApusHipKvCache *c, size_t B, const int32_t *rows, const int32_t *cu,

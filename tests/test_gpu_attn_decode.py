@@ -74,6 +74,54 @@ def test_decode_split_boundaries(hip, orc):
     _run(hip, orc, np.random.default_rng(2), cu, [1020, 1023, 1024, 2046, 3000], 3072)
 
 
+@pytest.mark.parametrize("pos0,k", [(0, 1), (15, 4), (16, 2), (63, 1), (64, 3), (60, 4),
+                                    (2047, 2), (2100, 3), (20001, 1), (9000, 4)])
+def test_decode_one_sequence(hip, orc, pos0, k):
+    """One sequence (k_attn_scores_few): keys that end inside a wavefront's
+    16 and inside a 64-key group, a group cut by the causal mask, one row
+    block and two, and pairs of few and of hundreds of runs (one wavefront
+    or four sum a row's partials)."""
+    _run(hip, orc, np.random.default_rng(pos0 + k), [0, k], [pos0], (pos0 + k + 31) // 32 * 32)
+
+
+def test_decode_few_and_ring_kernels_agree(hip):
+    """The same sequences in a call of few keys and in one with a long
+    sequence added that takes it past k_attn_scores_few's limit: both
+    within bf16 rounding and rounding flips of each other."""
+    import torch
+    dims = synth.ATTN_DIMS
+    nh, nkv, d, rot, theta = dims
+    rng = np.random.default_rng(4)
+    k = [1, 4, 2, 3, 1, 1, 2, 1]
+    pos0 = [30000, 29000, 8191, 33, 32500, 30001, 27777, 260000]
+    B = len(k)
+    cu = np.concatenate([[0], np.cumsum(k)]).astype(np.int32)
+    nblk = [-(-(p + n) // 32) for p, n in zip(pos0, k)]
+    ids = rng.permutation(sum(nblk)).astype(np.int32)
+    table = np.zeros((B, max(nblk)), np.int32)
+    for s in range(B):
+        table[s, :nblk[s]], ids = ids[:nblk[s]], ids[nblk[s]:]
+    dev = torch.device("cuda")
+    td = lambda a: torch.from_numpy(np.ascontiguousarray(a).view(np.int16)).to(dev)
+    g = torch.Generator(device=dev).manual_seed(4)
+    kc = torch.randn((sum(nblk), nkv, 32, d), generator=g, device=dev).to(torch.bfloat16)
+    vc = torch.randn((sum(nblk), nkv, d, 32), generator=g, device=dev).to(torch.bfloat16)
+    tab = torch.from_numpy(table).to(dev)
+    kv = hip.KvCache(kc.data_ptr(), vc.data_ptr(), tab.data_ptr(), table.shape[1], B, None)
+    layer = hip.attn_layer(dims, {n: td(v) for n, v in synth.attn_weights(rng).items()})
+    t = {n: td(v) for n, v in synth.attn_tokens(rng, int(cu[-1])).items()}
+    keys = lambda n: hip.attn_split_check(cu[:n + 1], pos0[:n])["writer_groups"] * 64
+    assert keys(B - 1) <= 8192 * 64 < keys(B)
+    ys = []
+    for n in (B - 1, B):
+        y = torch.zeros((int(cu[n]), nh * d), dtype=torch.bfloat16, device=dev)
+        hip.attn_decode_paged(layer, np.arange(n), cu[:n + 1], pos0[:n], t["qg"], t["k"], t["v"], kv, y)
+        ys.append(y[:int(cu[B - 1])].double())
+    torch.cuda.synchronize()
+    assert torch.isfinite(ys[0]).all()
+    assert float((ys[0] - ys[1]).norm() / ys[1].norm()) <= 2e-3
+
+
 def test_decode_config2_shape(hip, orc):
     """BASELINE config 2 per sequence: 32K-token cache, one new token
     (two sequences here; the bench runs 64)."""
