@@ -115,6 +115,7 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
 }
 __device__ __forceinline__ float rnd_hw(float x) { return (float)(__bf16)x; }
+__device__ __forceinline__ uint16_t bf_hw(float x) { return __builtin_bit_cast(uint16_t, (__bf16)x); }
 
 // max / sum of x over lanes l and l ^ 32, in both (v_permlane32_swap
 // exchanges one half of its two operands; with both = x the two results
@@ -615,7 +616,7 @@ __global__ __launch_bounds__(64 * NW) void k_attn_fa(
         const float rr = 1.0f / sqrtf(ss / (float)D + 1e-6f);
         // normed value of dim e of the lane's chunk ks
         auto nrm = [&](const u16x8 &xk, int e, const u16x8 &wv) {
-            return rndf((bf2f(xk[e]) * rr) * (1.0f + bf2f(wv[e])));
+            return rnd_hw((bf2f(xk[e]) * rr) * (1.0f + bf2f(wv[e])));
         };
         auto ldx = [&](int ks) { return *reinterpret_cast<const u16x8 *>(xr + ks * 16); };
         const uint16_t *cs = rope + (size_t)(qpos0 + tq) * (2 * R);
@@ -632,8 +633,8 @@ __global__ __launch_bounds__(64 * NW) void k_attn_fa(
             for (int e = 0; e < 8; e++) {
                 const float a = nrm(x0, e, w0), b = nrm(x1, e, w1);
                 const float cc = bf2f(cv[e]), sn = bf2f(sv[e]);
-                lo[e] = f2bf(rndf(a * cc) + rndf(-b * sn));     // dim d < 32
-                hi[e] = f2bf(rndf(b * cc) + rndf(a * sn));      // dim d + 32
+                lo[e] = bf_hw(rnd_hw(a * cc) + rnd_hw(-b * sn));     // dim d < 32
+                hi[e] = bf_hw(rnd_hw(b * cc) + rnd_hw(a * sn));      // dim d + 32
             }
             q[ks] = __builtin_bit_cast(bf16x8, lo);
             q[ks + 2] = __builtin_bit_cast(bf16x8, hi);
@@ -644,7 +645,7 @@ __global__ __launch_bounds__(64 * NW) void k_attn_fa(
             const u16x8 xk = ldx(ks);
             u16x8 out;
 #pragma unroll
-            for (int e = 0; e < 8; e++) out[e] = f2bf(nrm(xk, e, wv));
+            for (int e = 0; e < 8; e++) out[e] = bf_hw(nrm(xk, e, wv));
             q[ks] = __builtin_bit_cast(bf16x8, out);
         }
     }
@@ -733,20 +734,40 @@ __global__ __launch_bounds__(64 * NW) void k_attn_fa(
         const size_t row = (size_t)(tb + tk) * nh + head;
         const uint16_t *gr = qg + row * 2 * D + D;
         uint16_t *yr = y + row * D;
+        // rnd(sigmoid(gate)) by formula; where its rounding is in doubt (within
+        // 16 ulps of a midpoint, one code in 2000) or |gate| > 16, from the
+        // bf16-code table, which holds the reference's value. Gathering every
+        // code (64 distinct lines an instruction) held the address unit (one
+        // full tile alone: 47.4 -> 37.9 us; T = 1024 101 -> 92, 8192 785 -> 771).
 #pragma unroll
         for (int mt = 0; mt < D / 32; mt++) {
+            u16x4 gv[4], sg[4];
+            uint32_t doubt = 0;                // bit 15 - (4 q4 + i)
 #pragma unroll
-            for (int q4 = 0; q4 < 4; q4++) {
-                const int d0 = mt * 32 + 8 * q4 + 4 * c.h;
-                const u16x4 gv = *reinterpret_cast<const u16x4 *>(gr + d0);
-                u16x4 out;
+            for (int q4 = 0; q4 < 4; q4++)
+                gv[q4] = *reinterpret_cast<const u16x4 *>(gr + mt * 32 + 8 * q4 + 4 * c.h);
+#pragma unroll
+            for (int q4 = 0; q4 < 4; q4++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const float ov = rndf(o[mt][4 * q4 + i]);
-                    const float gs = bf2f(sig_bf[gv[i]]);     // rnd(sigmoid(gate))
-                    out[i] = f2bf(ov * gs);
+                    const float g = bf2f(gv[q4][i]);
+                    const float p = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.44269504088896341f));
+                    const bool far = (__float_as_uint(p) << 16) + 0x80100000u >= 0x210000u;
+                    doubt = doubt + doubt + (far && (gv[q4][i] & 0x7fff) <= 0x4180 ? 0u : 1u);
+                    sg[q4][i] = bf_hw(p);
                 }
-                *reinterpret_cast<u16x4 *>(yr + d0) = out;
+            if (__builtin_amdgcn_ballot_w64(doubt != 0)) {
+#pragma unroll
+                for (int e = 0; e < 16; e++)
+                    if (doubt >> (15 - e) & 1u) sg[e >> 2][e & 3] = sig_bf[gv[e >> 2][e & 3]];
+            }
+#pragma unroll
+            for (int q4 = 0; q4 < 4; q4++) {
+                u16x4 out;
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    out[i] = bf_hw(rnd_hw(o[mt][4 * q4 + i]) * bf2f(sg[q4][i]));
+                *reinterpret_cast<u16x4 *>(yr + mt * 32 + 8 * q4 + 4 * c.h) = out;
             }
         }
         // (trace) rnd(o) before the gate, in a loop of its own: a

@@ -89,6 +89,33 @@ def test_prefill_score_growth(hip, orc):
          edit=edit)
 
 
+def test_prefill_gate_every_code(hip):
+    """The flash kernel's output gate on every bf16 code (by formula, from
+    the table where that is in doubt): 16 one-token sequences whose v is 1,
+    so that P = 1, o = 1 and y = rnd(sigmoid(gate)), bit for bit what the
+    outgate op gives."""
+    import torch
+    dims = synth.ATTN_DIMS
+    nh, nkv, d, rot, theta = dims
+    rng = np.random.default_rng(21)
+    B = 16
+    tok = synth.attn_tokens(rng, B)
+    codes = np.arange(1 << 16, dtype=np.uint32).astype(np.uint16)
+    codes[(codes & 0x7FFF) > 0x7F80] = 0            # NaN
+    codes = rng.permutation(codes)
+    tok["qg"][:, :, d:] = codes.reshape(B, nh, d)
+    tok["v"][:] = 0x3F80
+    layer = hip.attn_layer(dims, {k: _td(torch, v) for k, v in synth.attn_weights(rng).items()})
+    t = {k: _td(torch, v) for k, v in tok.items()}
+    dk = torch.zeros((B, nkv, 32, d), dtype=torch.int16, device="cuda")
+    dv = torch.zeros((B, nkv, 1, d, 32), dtype=torch.int16, device="cuda")
+    y = torch.empty((B, nh * d), dtype=torch.int16, device="cuda")
+    hip.attn_prefill(layer, np.arange(B + 1), np.zeros(B), t["qg"], t["k"], t["v"], dk, dv, 32, y)
+    torch.cuda.synchronize()
+    want = hip.attn_outgate(np.full(1 << 16, 0x3F80, np.uint16), codes)
+    assert np.array_equal(y.cpu().numpy().view(np.uint16).ravel(), want)
+
+
 def test_prefill_long_prefix(hip, orc):
     """A continuation after a 30,000-position cached prefix: RoPE at large
     positions in the flash kernel's own q rows, and ~470 key tiles per
