@@ -793,6 +793,77 @@ __global__ __launch_bounds__(64 * NW) void k_attn_fa(
 
 namespace apus {
 
+// Short continuations of long prefixes (the next turn of a long chat). A
+// query tile of 32 tokens walks all its keys on one CU, twice, so a few new
+// tokens after a long prefix take as long as a full tile while most CUs
+// idle: 13 tokens after 8000 positions 497 us. Such a sequence can run
+// through the split-K decode kernels instead, 4 tokens at a time (pieces
+// that share a block-table row): 40 us. The times below are fits of both,
+// in us (FA: 30 + 3.7 per 64-key tile of the longest row, tiles beside
+// each other; decode: 18 + 0.0155 per 64 keys of a piece and kv head).
+struct Short {
+    size_t first, last;                // sequences first .. last
+    size_t pieces;
+    double groups;                     // 64-key groups over pieces and kv heads
+};
+static double fa_us(int64_t keys) { return 30.0 + 3.7 * (double)((keys + KT - 1) / KT); }
+// A sequence is short by its own sizes alone (so it goes the same way in
+// any batch that is not much larger): a prefix of at least 512 positions
+// and four times the new tokens, and less than half the time.
+static bool short_seq(int64_t n, int64_t pos0, size_t nkv, double *groups) {
+    if (n < 1 || pos0 < 512 || pos0 < 4 * n) return false;
+    *groups = (double)((n + 3) / 4) * (double)nkv * (double)((pos0 + n + 63) / 64);
+    return 18.0 + 0.0155 * *groups < 0.5 * fa_us(pos0 + n);
+}
+// The runs of short sequences to take out of the flash kernel's grid: all or
+// none, if that saves more than it costs. Bounds: one call's by-value
+// metadata, and 100 MB of scores in library scratch.
+constexpr double kShortGroups = 24576.0;
+static std::vector<Short> short_runs(size_t B, const int32_t *cu, const int32_t *pos0, size_t nkv) {
+    std::vector<Short> runs;
+    double groups = 0.0, t_short = 0.0, t_rest = 0.0, sum = 0.0;
+    size_t pieces = 0;
+    for (size_t s = 0; s < B; s++) {
+        const int64_t n = cu[s + 1] - cu[s];
+        double g = 0.0;
+        if (short_seq(n, pos0[s], nkv, &g)) {
+            if (runs.empty() || runs.back().last + 1 != s) runs.push_back(Short{s, s, 0, 0.0});
+            runs.back().last = s;
+            runs.back().pieces += (size_t)(n + 3) / 4;
+            runs.back().groups += g;
+            groups += g;
+            pieces += (size_t)(n + 3) / 4;
+            t_short = std::max(t_short, fa_us(pos0[s] + n));
+        } else if (n > 0) {
+            t_rest = std::max(t_rest, fa_us(pos0[s] + n));
+            sum += (double)nkv * (double)((n + TQ - 1) / TQ) * (fa_us(pos0[s] + n / 2) - 20.0);
+        }
+    }
+    t_rest = std::max(t_rest, sum / (double)cu_count());
+    if (pieces > (size_t)kAttnInlineSeqs || groups > kShortGroups ||
+        18.0 * (double)runs.size() + 0.0155 * groups > 0.8 * (t_short - t_rest))
+        runs.clear();
+    return runs;
+}
+// The sequences of r as pieces of at most 4 tokens through the decode path.
+// (Every piece's k and v rows are in the cache before any piece's scores.)
+static int short_run(const Short &r, const ApusHipAttnLayer *L, const int32_t *cu,
+                     const int32_t *pos0, const int32_t *rows, const uint16_t *qg,
+                     const uint16_t *k, const uint16_t *v, const KvRef &kv, uint16_t *y) {
+    std::vector<int32_t> pcu{0}, ppos, prow;
+    const int32_t t0 = cu[r.first];
+    for (size_t s = r.first; s <= r.last; s++)
+        for (int32_t t = cu[s]; t < cu[s + 1]; t += 4) {
+            pcu.push_back(std::min(t + 4, cu[s + 1]) - t0);
+            ppos.push_back(pos0[s] + (t - cu[s]));
+            prow.push_back(rows ? rows[s] : (int32_t)s);
+        }
+    const size_t qd = L->nh * D, kd = L->nkv * D;
+    return attn_decode_kv(L, ppos.size(), pcu.data(), ppos.data(), prow.data(),
+                          qg + (size_t)t0 * 2 * qd, k + (size_t)t0 * kd, v + (size_t)t0 * kd, kv,
+                          y + (size_t)t0 * qd);
+}
+
 int attn_prefill_kv(const ApusHipAttnLayer *L, size_t B, const int32_t *cu, const int32_t *pos0,
                     const int32_t *rows, const uint16_t *qg, const uint16_t *k,
                     const uint16_t *v, const KvRef &kv, uint16_t *y) {
@@ -807,6 +878,14 @@ int attn_prefill_kv(const ApusHipAttnLayer *L, size_t B, const int32_t *cu, cons
         return r;
     const size_t Ttot = (size_t)cu[B];
     if (Ttot == 0) return kOk;
+    // (a trace's buffers are indexed by the call's tokens: not in pieces)
+    std::vector<Short> shorts;
+    if (!attn_trace()) shorts = short_runs(B, cu, pos0, L->nkv);
+    auto is_short = [&](size_t s) {
+        for (const Short &r : shorts)
+            if (s >= r.first && s <= r.last) return true;
+        return false;
+    };
     size_t max_pos = 0;
     std::vector<int32_t> meta(4 * B + 2);
     int32_t *mcu = meta.data(), *mpos = mcu + B + 1, *mtoff = mpos + B, *mhd = mtoff + B + 1;
@@ -814,12 +893,15 @@ int attn_prefill_kv(const ApusHipAttnLayer *L, size_t B, const int32_t *cu, cons
     for (size_t s = 0; s < B; s++) {
         const int32_t ns = cu[s + 1] - cu[s];
         max_pos = std::max(max_pos, (size_t)pos0[s] + (size_t)ns);
-        mtoff[s + 1] = mtoff[s] + (ns + TQ - 1) / TQ;
+        mtoff[s + 1] = mtoff[s] + (is_short(s) ? 0 : (ns + TQ - 1) / TQ);
         mhd[s] = rows ? rows[s] : (int32_t)s;
     }
     memcpy(mcu, cu, (B + 1) * 4);
     memcpy(mpos, pos0, B * 4);
     const size_t ntiles = (size_t)mtoff[B];
+    for (const Short &r : shorts)
+        if (int e = short_run(r, L, cu, pos0, rows, qg, k, v, kv, y)) return e;
+    if (ntiles == 0) return kOk;
     FaSeqs fs;
     fs.n = (int32_t)B;
     const int32_t *fdm = nullptr;

@@ -140,6 +140,19 @@ def test_prefill_tile_edges(hip, orc):
     _run(hip, orc, np.random.default_rng(12), cu, [0, 31, 32, 63, 5, 100], 160, tag="edges")
 
 
+@pytest.mark.parametrize("lens,pos0", [
+    ([13], [1900]),                         # alone: no flash tile is left
+    ([40, 5, 13, 1, 0, 4, 200], [3, 2000, 1500, 512, 90, 3000, 700]),   # one run and a lone one
+    ([2, 300, 17], [2500, 64, 4000])])      # on either side of a prompt
+def test_prefill_short_continuations(hip, orc, lens, pos0):
+    """Few new tokens after a long prefix, which run as pieces of 4 tokens
+    through the decode kernels beside the flash kernel's sequences: piece
+    remainders, an empty sequence among them, pieces of two sequences in
+    one call."""
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    _run(hip, orc, np.random.default_rng(len(lens)), cu, pos0, 4032, tag="short")
+
+
 def test_prefill_long(hip, orc):
     """One 2048-token causal prefill from position 0 (config 3's shape at a
     quarter of its length)."""
