@@ -149,6 +149,96 @@ __global__ __launch_bounds__(64) void k_gemm_seq(const uint16_t *__restrict__ w,
     if (o < O) y[(size_t)m * O + o] = f2bf(acc);
 }
 
+// The same sums for K a multiple of 64 (up to 16384): 64 outputs of R rows
+// (1 .. 4) a workgroup. Wavefront r < R runs row r's 64 chains, a lane each,
+// and four more stream the weights for all rows, widen them and lay them in
+// LDS as the chains read them. In k_gemm_seq a wavefront does all of this
+// for one row, so that a k costs it 2.5 instructions besides the wait for
+// the sum before it, its loads are 16-byte pieces of 64 rows, and the weights
+// are read once per row. 12352 x 2048: one row 18.0 -> 16.3 us, 3 rows 30.2 ->
+// 19.5, 8 rows 72 -> 31; 2048 x 4096 33.1 -> 27.2. What is left is the chain:
+// 6 ns a k (reads placed between its multiply-adds, or a part ahead of them,
+// made that 6.5 to 6.9).
+constexpr int kSeqK = 64;                  // k per chunk
+constexpr int kSeqDepth = 8;               // chunks in flight per loader
+__global__ __launch_bounds__(512) void k_gemm_seq64(const uint16_t *__restrict__ w,
+                                                    const uint16_t *__restrict__ x,
+                                                    uint16_t *__restrict__ y, int M, int O, int K,
+                                                    int R) {
+    // chunk buffers [k / 4][row][4] (PITCH: 16 rows of padding spread a
+    // loader's 8 pieces of a row over the banks), then x as fp32
+    constexpr int PITCH = 64 * 4 + 4;
+    __shared__ __attribute__((aligned(16))) float wl[2][(kSeqK / 4) * PITCH];
+    extern __shared__ __attribute__((aligned(16))) float4 xf[];
+    const int m0 = blockIdx.y * R, o0 = blockIdx.x * 64, nch = K / kSeqK;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int e = threadIdx.x; e < R * (K / 8); e += 64 * (4 + R)) {   // x rows (past M: the last)
+        const int r = e / (K / 8), i = e % (K / 8);
+        const u16x8 v = reinterpret_cast<const u16x8 *>(x + (size_t)min(m0 + r, M - 1) * K)[i];
+        xf[2 * e] = make_float4(bf2f(v[0]), bf2f(v[1]), bf2f(v[2]), bf2f(v[3]));
+        xf[2 * e + 1] = make_float4(bf2f(v[4]), bf2f(v[5]), bf2f(v[6]), bf2f(v[7]));
+    }
+    if (wave >= R) {
+        // loader: rows r0 + lane / 8 and that + 8, 16-byte piece lane % 8 of
+        // each chunk's 128 bytes. Loads past the last chunk read it again.
+        const int r0 = (wave - R) * 16 + (lane >> 3), pc = lane & 7;
+        const u16x8 *src[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+            src[i] = reinterpret_cast<const u16x8 *>(w + (size_t)min(o0 + r0 + 8 * i, O - 1) * K) + pc;
+        u16x8 q[kSeqDepth][2];
+        auto load = [&](int c, u16x8 (&d)[2]) {
+#pragma unroll
+            for (int i = 0; i < 2; i++) d[i] = src[i][min(c, nch - 1) * (kSeqK / 8)];
+        };
+        auto put = [&](int c, const u16x8 (&d)[2]) {
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                float *p = wl[c & 1] + 2 * pc * PITCH + (r0 + 8 * i) * 4;
+                *reinterpret_cast<float4 *>(p) = make_float4(bf2f(d[i][0]), bf2f(d[i][1]), bf2f(d[i][2]), bf2f(d[i][3]));
+                *reinterpret_cast<float4 *>(p + PITCH) = make_float4(bf2f(d[i][4]), bf2f(d[i][5]), bf2f(d[i][6]), bf2f(d[i][7]));
+            }
+        };
+#pragma unroll
+        for (int c = 0; c < kSeqDepth; c++) load(c, q[c]);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        for (int c0 = 0; c0 < nch; c0 += kSeqDepth) {
+#pragma unroll
+            for (int j = 0; j < kSeqDepth; j++) {
+                const int c = c0 + j;
+                if (c < nch) {
+                    // (this buffer's readers passed the barrier of chunk c - 1)
+                    put(c, q[j]);
+                    load(c + kSeqDepth, q[j]);
+                    // keep the loads here (they would be sunk to their use)
+                    asm volatile("" ::: "memory");
+                    __builtin_amdgcn_sched_barrier(0);
+                    __syncthreads();               // chunk c is in place
+                }
+            }
+        }
+        return;
+    }
+    const float4 *xc = xf + wave * (K / 4);
+    float acc = 0.0f;
+    for (int c = 0; c < nch; c++) {
+        __syncthreads();                           // chunk c is in place
+        const float4 *wc = reinterpret_cast<const float4 *>(wl[c & 1]) + lane;
+#pragma unroll
+        for (int i = 0; i < kSeqK / 4; i++) {
+            const float4 a = wc[i * (PITCH / 4)], b = xc[c * (kSeqK / 4) + i];
+            acc = fmaf(a.x, b.x, acc);
+            acc = fmaf(a.y, b.y, acc);
+            acc = fmaf(a.z, b.z, acc);
+            acc = fmaf(a.w, b.w, acc);
+        }
+    }
+    const int m = m0 + wave;
+    if (m < M && o0 + lane < O) y[(size_t)m * O + o0 + lane] = f2bf(acc);
+}
+
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -796,7 +886,15 @@ int launch_seq(const uint16_t *w, const uint16_t *x, uint16_t *y, size_t M, size
     const dim3 grid(cdiv(O, 64), (unsigned)M);
     if (vec) {
         if (K * 2 > 64 * 1024) return set_error(kErrUnsupported, "sequential gemm takes K up to 32768");
-        if (K * 4 <= 64 * 1024)
+        // rows per workgroup: no more than give every CU one (a chain that
+        // shares its SIMD with another is slower: 4 x 8192 x 2048 20.0 us with
+        // four, 16.8 with two), x rows as fp32 in at most 64 KiB of LDS
+        const int R = (int)std::min<size_t>({M, 4, 16384 / K, cdiv(cdiv(O, 64) * M, cu_count())});
+        if (K % kSeqK == 0 && R > 0)
+            APUS_TIMED("k_gemm_seq",
+                       k_gemm_seq64<<<dim3(grid.x, cdiv(M, R)), 64 * (4 + R), R * K * 4, stream()>>>(
+                           w, x, y, (int)M, (int)O, (int)K, R));
+        else if (K * 4 <= 64 * 1024)
             APUS_TIMED("k_gemm_seq",
                        k_gemm_seq<true, true><<<grid, 64, K * 4, stream()>>>(w, x, y, (int)O, (int)K));
         else

@@ -63,6 +63,23 @@ def test_gemm_dev_bitwise(hip, orc, M, O, K):
     assert np.array_equal(y.cpu().numpy().view(np.uint16), orc.bf16_gemm(w, x))
 
 
+# K a multiple of 64 (weights streamed by wavefronts of their own): one
+# chunk, fewer chunks than are kept in flight, one more; one to four rows a
+# workgroup with a remainder; outputs past a workgroup's 64; the largest K
+@pytest.mark.parametrize("M,O,K", [(1, 64, 64), (5, 70, 128), (3, 4100, 576), (2, 65, 16384),
+                                   (7, 12352, 512), (11, 8200, 192), (1, 130, 16448)])
+def test_gemm_dev_bitwise_chunks(hip, orc, M, O, K):
+    import torch
+    rng = np.random.default_rng(M * O + K)
+    w = synth.normal_bf16(rng, (O, K), K ** -0.5)
+    x = synth.normal_bf16(rng, (M, K))
+    print(f"[proj] chunks M={M} O={O} K={K}", flush=True)
+    y = torch.empty((M, O), dtype=torch.int16, device="cuda")
+    hip.bf16_gemm_dev(_dev(torch, w), _dev(torch, x), y, exact=True)
+    torch.cuda.synchronize()
+    assert np.array_equal(y.cpu().numpy().view(np.uint16), orc.bf16_gemm(w, x))
+
+
 def test_gemm_dev_bitwise_wide_range(hip, orc):
     """Operands whose magnitudes span 2^-60 .. 2^60 (every product still in
     fp32's normal range): the sequential kernel's fused multiply-add rounds
