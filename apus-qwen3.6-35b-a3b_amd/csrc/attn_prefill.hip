@@ -3,12 +3,13 @@
 // causal GQA over the cache, sigmoid output gate) for B sequences of any
 // length, with the attention as an MFMA flash-attention kernel.
 //
-// k_attn_fa: one workgroup of 8 wavefronts (two per SIMD) per (32-token
-// query tile, kv head), tiles dealt longest first. The 8 q heads of the
-// kv head x 32 tokens are 256 query rows; wavefront w owns tokens
-// 4w..4w+3 (32 rows: one MFMA N-tile), its Q rows held in registers. It
-// forms those rows itself from the layer input ((1+w) RMSNorm, RoPE);
-// k_attn_prep forms the k rows and appends k and v to the cache.
+// k_attn_fa (k_attn_fa16, below, for calls of few tiles): one workgroup of 8
+// wavefronts (two per SIMD) per (32-token query tile, kv head), tiles dealt
+// longest first. The 8 q heads of the kv head x 32 tokens are 256 query
+// rows; wavefront w owns tokens 4w..4w+3 (32 rows: one MFMA N-tile), its Q
+// rows held in registers. It forms those rows itself from the layer input
+// ((1+w) RMSNorm, RoPE); k_attn_prep forms the k rows and appends k and v to
+// the cache.
 //
 // The attention runs over the keys twice:
 //   pass 1: S^T = K Q^T on MFMA 32x32x16 bf16 (fp32 accumulation); with
@@ -58,6 +59,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/apus_hip.h"
@@ -398,7 +400,8 @@ __device__ __forceinline__ void fa_p1_step(const FaCtx &c, int Kn, int kj,
         ps = 0.0f;
 #pragma unroll
         for (int i = 0; i < 16; i++) ps += e[i];
-        w.lsum = w.lsum * __builtin_amdgcn_exp2f((w.M - mn) * c.c2) + sum32(ps);
+        // (a row with no key yet in a wavefront whose other rows have: 0)
+        w.lsum = mn > -INFINITY ? w.lsum * __builtin_amdgcn_exp2f((w.M - mn) * c.c2) + sum32(ps) : 0.0f;
         w.M = mn;
     } else {
         w.lsum = ls;
@@ -470,10 +473,161 @@ __device__ __forceinline__ void fa_pv_last(const FaCtx &c, int Vp, const bf16x8 
     }
 }
 
+// pass 2's K2 of two sets of scores' (M, s)
+__device__ __forceinline__ float fa_join(float m0, float s0, float m1, float s1, float c2) {
+    const float m = fmaxf(m0, m1);
+    const float s = s0 * __builtin_amdgcn_exp2f((m0 - m) * c2) + s1 * __builtin_amdgcn_exp2f((m1 - m) * c2);
+    return m * c2 + __builtin_amdgcn_logf(s);  // v_log_f32: log2
+}
+
 // wait for this wavefront's copies, then the barrier that publishes them
 __device__ __forceinline__ void fa_publish() {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
+}
+
+// The q row, formed here from the layer's input as k_attn_prep forms k
+// (c/attn.h:175-236 via c/layer.h:300-312): (1+w) RMSNorm with the
+// ascending sum of squares, then NeoX RoPE on dims 0..63 at the token's
+// position, each product rounded as the reference rounds it. The lane
+// holds dims 16 ks + 8 h .. +7, and lane l ^ 32 the other 8 of each 16;
+// each lane takes its partner's chunks by exchange and runs the whole
+// ascending sum over the 32 8-dim chunks itself. A RoPE pair (d, d + 32)
+// lies in chunks ks and ks + 2 of the same lane.
+__device__ __forceinline__ void fa_q(const FaCtx &c, const uint16_t *__restrict__ xr,
+                                     const uint16_t *__restrict__ qn_w,
+                                     const uint16_t *__restrict__ rope, int pos,
+                                     bf16x8 (&q)[D / 16]) {
+    constexpr int R = 32;                  // rotary pairs (64 rotated dims)
+    xr += c.h * 8;
+    float ss = 0.0f;
+    {
+        u16x8 xv[D / 16];
+#pragma unroll
+        for (int ks = 0; ks < D / 16; ks++) xv[ks] = *reinterpret_cast<const u16x8 *>(xr + ks * 16);
+        // the other half's chunks (independent exchanges, all in flight
+        // together); then both halves run the whole chain, in order
+        u16x8 px[D / 16];
+#pragma unroll
+        for (int ks = 0; ks < D / 16; ks++) {
+            const uint4 u = __builtin_bit_cast(uint4, xv[ks]);
+            px[ks] = __builtin_bit_cast(u16x8, make_uint4(__shfl_xor(u.x, 32), __shfl_xor(u.y, 32),
+                                                          __shfl_xor(u.z, 32), __shfl_xor(u.w, 32)));
+        }
+#pragma unroll
+        for (int ks = 0; ks < D / 16; ks++) {
+#pragma unroll
+            for (int hh = 0; hh < 2; hh++) {
+                const u16x8 xc = hh == c.h ? xv[ks] : px[ks];   // chunk (ks, hh)
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const float f = bf2f(xc[e]);
+                    ss = fmaf(f, f, ss);   // f * f exact: bf16 squared
+                }
+            }
+        }
+    }
+    // the row is read again below, a chunk at a time (an L2 hit), so
+    // that the 64 registers of the first read are not live beside q
+    asm volatile("" ::: "memory");
+    const float rr = 1.0f / sqrtf(ss / (float)D + 1e-6f);
+    // normed value of dim e of the lane's chunk ks
+    auto nrm = [&](const u16x8 &xk, int e, const u16x8 &wv) {
+        return rnd_hw((bf2f(xk[e]) * rr) * (1.0f + bf2f(wv[e])));
+    };
+    auto ldx = [&](int ks) { return *reinterpret_cast<const u16x8 *>(xr + ks * 16); };
+    const uint16_t *cs = rope + (size_t)pos * (2 * R);
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) {
+        const u16x8 w0 = *reinterpret_cast<const u16x8 *>(qn_w + ks * 16 + c.h * 8);
+        const u16x8 w1 = *reinterpret_cast<const u16x8 *>(qn_w + (ks + 2) * 16 + c.h * 8);
+        const int i0 = ks * 16 + c.h * 8;          // pair index of the chunk's first dim
+        const u16x8 cv = *reinterpret_cast<const u16x8 *>(cs + i0);
+        const u16x8 sv = *reinterpret_cast<const u16x8 *>(cs + R + i0);
+        const u16x8 x0 = ldx(ks), x1 = ldx(ks + 2);
+        u16x8 lo, hi;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float a = nrm(x0, e, w0), b = nrm(x1, e, w1);
+            const float cc = bf2f(cv[e]), sn = bf2f(sv[e]);
+            lo[e] = bf_hw(rnd_hw(a * cc) + rnd_hw(-b * sn));     // dim d < 32
+            hi[e] = bf_hw(rnd_hw(b * cc) + rnd_hw(a * sn));      // dim d + 32
+        }
+        q[ks] = __builtin_bit_cast(bf16x8, lo);
+        q[ks + 2] = __builtin_bit_cast(bf16x8, hi);
+    }
+#pragma unroll
+    for (int ks = 4; ks < D / 16; ks++) {
+        const u16x8 wv = *reinterpret_cast<const u16x8 *>(qn_w + ks * 16 + c.h * 8);
+        const u16x8 xk = ldx(ks);
+        u16x8 out;
+#pragma unroll
+        for (int e = 0; e < 8; e++) out[e] = bf_hw(nrm(xk, e, wv));
+        q[ks] = __builtin_bit_cast(bf16x8, out);
+    }
+}
+
+// Epilogue of a query row's dims d0 .. d0 + 32 NMT - 1: o = rnd(O);
+// y = rnd(o * rnd(sigmoid(gate)))
+template <int NMT>
+__device__ __forceinline__ void fa_out(const FaCtx &c, const f32x16 (&o)[NMT], size_t row, int d0,
+                                       const uint16_t *__restrict__ qg, uint16_t *__restrict__ y,
+                                       const uint16_t *__restrict__ sig_bf,
+                                       uint16_t *__restrict__ tr_attno) {
+    const uint16_t *gr = qg + row * 2 * D + D + d0;
+    uint16_t *yr = y + row * D + d0;
+    // rnd(sigmoid(gate)) by formula; where its rounding is in doubt (within
+    // 16 ulps of a midpoint, one code in 2000) or |gate| > 16, from the
+    // bf16-code table, which holds the reference's value. Gathering every
+    // code (64 distinct lines an instruction) held the address unit (one
+    // full tile alone: 47.4 -> 37.9 us; T = 1024 101 -> 92, 8192 785 -> 771).
+#pragma unroll
+    for (int mt = 0; mt < NMT; mt++) {
+        u16x4 gv[4], sg[4];
+        uint32_t doubt = 0;                // bit 15 - (4 q4 + i)
+#pragma unroll
+        for (int q4 = 0; q4 < 4; q4++)
+            gv[q4] = *reinterpret_cast<const u16x4 *>(gr + mt * 32 + 8 * q4 + 4 * c.h);
+#pragma unroll
+        for (int q4 = 0; q4 < 4; q4++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float g = bf2f(gv[q4][i]);
+                const float p = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.44269504088896341f));
+                const bool far = (__float_as_uint(p) << 16) + 0x80100000u >= 0x210000u;
+                doubt = doubt + doubt + (far && (gv[q4][i] & 0x7fff) <= 0x4180 ? 0u : 1u);
+                sg[q4][i] = bf_hw(p);
+            }
+        if (__builtin_amdgcn_ballot_w64(doubt != 0)) {
+#pragma unroll
+            for (int e = 0; e < 16; e++)
+                if (doubt >> (15 - e) & 1u) sg[e >> 2][e & 3] = sig_bf[gv[e >> 2][e & 3]];
+        }
+#pragma unroll
+        for (int q4 = 0; q4 < 4; q4++) {
+            u16x4 out;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                out[i] = bf_hw(rnd_hw(o[mt][4 * q4 + i]) * bf2f(sg[q4][i]));
+            *reinterpret_cast<u16x4 *>(yr + mt * 32 + 8 * q4 + 4 * c.h) = out;
+        }
+    }
+    // (trace) rnd(o) before the gate, in a loop of its own: a
+    // conditional store inside the loop above would make the compiler
+    // drain the memory counter at every join
+    if (tr_attno) {
+#pragma unroll
+        for (int mt = 0; mt < NMT; mt++) {
+#pragma unroll
+            for (int q4 = 0; q4 < 4; q4++) {
+                const int d = d0 + mt * 32 + 8 * q4 + 4 * c.h;
+                u16x4 oc;
+#pragma unroll
+                for (int i = 0; i < 4; i++) oc[i] = f2bf(rndf(o[mt][4 * q4 + i]));
+                *reinterpret_cast<u16x4 *>(tr_attno + row * D + d) = oc;
+            }
+        }
+    }
 }
 
 __global__ __launch_bounds__(64 * NW) void k_attn_fa(
@@ -570,86 +724,12 @@ __global__ __launch_bounds__(64 * NW) void k_attn_fa(
 
     // query row of this lane: token 4w + l32/8, head l32%8 of the kv head
     const int tk = c.wave * 4 + c.l32 / GRP, head = kvh * GRP + c.l32 % GRP;
-    // The q row, formed here from the layer's input as k_attn_prep forms k
-    // (c/attn.h:175-236 via c/layer.h:300-312): (1+w) RMSNorm with the
-    // ascending sum of squares, then NeoX RoPE on dims 0..63 at the token's
-    // position, each product rounded as the reference rounds it. The lane
-    // holds dims 16 ks + 8 h .. +7, and lane l ^ 32 the other 8 of each 16;
-    // each lane takes its partner's chunks by exchange and runs the whole
-    // ascending sum over the 32 8-dim chunks itself. A RoPE pair (d, d + 32)
-    // lies in chunks ks and ks + 2 of the same lane.
     bf16x8 q[D / 16];
     {
-        constexpr int R = 32;                  // rotary pairs (64 rotated dims)
         const int tq = min(tk, nt - 1);
-        const uint16_t *xr = qg + ((size_t)(tb + tq) * nh + head) * 2 * D + c.h * 8;
-        float ss = 0.0f;
-        {
-            u16x8 xv[D / 16];
-#pragma unroll
-            for (int ks = 0; ks < D / 16; ks++) xv[ks] = *reinterpret_cast<const u16x8 *>(xr + ks * 16);
-            // the other half's chunks (independent exchanges, all in flight
-            // together); then both halves run the whole chain, in order
-            u16x8 px[D / 16];
-#pragma unroll
-            for (int ks = 0; ks < D / 16; ks++) {
-                const uint4 u = __builtin_bit_cast(uint4, xv[ks]);
-                px[ks] = __builtin_bit_cast(u16x8, make_uint4(__shfl_xor(u.x, 32), __shfl_xor(u.y, 32),
-                                                              __shfl_xor(u.z, 32), __shfl_xor(u.w, 32)));
-            }
-#pragma unroll
-            for (int ks = 0; ks < D / 16; ks++) {
-#pragma unroll
-                for (int hh = 0; hh < 2; hh++) {
-                    const u16x8 xc = hh == c.h ? xv[ks] : px[ks];   // chunk (ks, hh)
-#pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        const float f = bf2f(xc[e]);
-                        ss = fmaf(f, f, ss);   // f * f exact: bf16 squared
-                    }
-                }
-            }
-        }
-        // the row is read again below, a chunk at a time (an L2 hit), so
-        // that the 64 registers of the first read are not live beside q
-        asm volatile("" ::: "memory");
-        const float rr = 1.0f / sqrtf(ss / (float)D + 1e-6f);
-        // normed value of dim e of the lane's chunk ks
-        auto nrm = [&](const u16x8 &xk, int e, const u16x8 &wv) {
-            return rnd_hw((bf2f(xk[e]) * rr) * (1.0f + bf2f(wv[e])));
-        };
-        auto ldx = [&](int ks) { return *reinterpret_cast<const u16x8 *>(xr + ks * 16); };
-        const uint16_t *cs = rope + (size_t)(qpos0 + tq) * (2 * R);
-#pragma unroll
-        for (int ks = 0; ks < 2; ks++) {
-            const u16x8 w0 = *reinterpret_cast<const u16x8 *>(qn_w + ks * 16 + c.h * 8);
-            const u16x8 w1 = *reinterpret_cast<const u16x8 *>(qn_w + (ks + 2) * 16 + c.h * 8);
-            const int i0 = ks * 16 + c.h * 8;          // pair index of the chunk's first dim
-            const u16x8 cv = *reinterpret_cast<const u16x8 *>(cs + i0);
-            const u16x8 sv = *reinterpret_cast<const u16x8 *>(cs + R + i0);
-            const u16x8 x0 = ldx(ks), x1 = ldx(ks + 2);
-            u16x8 lo, hi;
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const float a = nrm(x0, e, w0), b = nrm(x1, e, w1);
-                const float cc = bf2f(cv[e]), sn = bf2f(sv[e]);
-                lo[e] = bf_hw(rnd_hw(a * cc) + rnd_hw(-b * sn));     // dim d < 32
-                hi[e] = bf_hw(rnd_hw(b * cc) + rnd_hw(a * sn));      // dim d + 32
-            }
-            q[ks] = __builtin_bit_cast(bf16x8, lo);
-            q[ks + 2] = __builtin_bit_cast(bf16x8, hi);
-        }
-#pragma unroll
-        for (int ks = 4; ks < D / 16; ks++) {
-            const u16x8 wv = *reinterpret_cast<const u16x8 *>(qn_w + ks * 16 + c.h * 8);
-            const u16x8 xk = ldx(ks);
-            u16x8 out;
-#pragma unroll
-            for (int e = 0; e < 8; e++) out[e] = bf_hw(nrm(xk, e, wv));
-            q[ks] = __builtin_bit_cast(bf16x8, out);
-        }
+        fa_q(c, qg + ((size_t)(tb + tq) * nh + head) * 2 * D, qn_w, rope, qpos0 + tq, q);
     }
-    FaRow w{qpos0 + tk, -INFINITY, 0.0f, 0.0f};
+    FaRow w{qpos0 + tk, -INFINITY, 0.0f, 0.0f}, w1 = w;   // of the even and of the odd 32-key steps
 
     // Tile u = 0 .. 2nkt-1 of the key stream: pass u / nkt, key tile
     // u % nkt. begin_tile(u) publishes tile u and starts the copy of u+1.
@@ -678,26 +758,26 @@ __global__ __launch_bounds__(64 * NW) void k_attn_fa(
     // a step with keys from kj needs the causal mask when it reaches past
     // this wavefront's first query
     const int qminw = qpos0 + 4 * c.wave;
-#define FA_P1(NEXT, Kn, kj)                                                    \
+#define FA_P1(NEXT, Kn, kj, row)                                               \
     do {                                                                       \
         const int kj_ = (kj);                                                  \
-        if (kj_ + 31 > qminw) fa_p1_step<NEXT, true>(c, Kn, kj_, q, sc, w);    \
-        else fa_p1_step<NEXT, false>(c, Kn, kj_, q, sc, w);                    \
+        if (kj_ + 31 > qminw) fa_p1_step<NEXT, true>(c, Kn, kj_, q, sc, row);  \
+        else fa_p1_step<NEXT, false>(c, Kn, kj_, q, sc, row);                  \
     } while (0)
 
     // pass 1 (steps j = 0 .. 2nkt-1; step j folds S(j) while S(j+1) is
     // formed)
     begin_tile(0);
     f32x16 sc = fa_s(c, kbuf(0), q);
-    FA_P1(true, kbuf(0) + HALF, 0);
+    FA_P1(true, kbuf(0) + HALF, 0, w);
     for (int u = 1; u < nkt; u++) {
         begin_tile(u);
-        FA_P1(true, kbuf(u), (u - 1) * KT + 32);
-        FA_P1(true, kbuf(u) + HALF, u * KT);
+        FA_P1(true, kbuf(u), (u - 1) * KT + 32, w1);
+        FA_P1(true, kbuf(u) + HALF, u * KT, w);
     }
     begin_tile(nkt);                     // pass 2's key tile 0 (and its V)
-    FA_P1(false, 0, (nkt - 1) * KT + 32);
-    w.K2 = w.M * c.c2 + __builtin_amdgcn_logf(w.lsum);     // v_log_f32: log2
+    FA_P1(false, 0, (nkt - 1) * KT + 32, w1);
+    w.K2 = fa_join(w.M, w.lsum, w1.M, w1.lsum, c.c2);
 
     // pass 2 (step j = 2kt + half of key tile kt, in stream tile nkt + kt)
     f32x16 o[D / 32];
@@ -729,64 +809,268 @@ __global__ __launch_bounds__(64 * NW) void k_attn_fa(
     fa_pv_last(c, vbuf(2 * nkt - 1, 1), pp, o);
 
 #undef FA_P1
-    // epilogue: o = rnd(O); y = rnd(o * rnd(sigmoid(gate)))
-    if (tk < nt) {
-        const size_t row = (size_t)(tb + tk) * nh + head;
-        const uint16_t *gr = qg + row * 2 * D + D;
-        uint16_t *yr = y + row * D;
-        // rnd(sigmoid(gate)) by formula; where its rounding is in doubt (within
-        // 16 ulps of a midpoint, one code in 2000) or |gate| > 16, from the
-        // bf16-code table, which holds the reference's value. Gathering every
-        // code (64 distinct lines an instruction) held the address unit (one
-        // full tile alone: 47.4 -> 37.9 us; T = 1024 101 -> 92, 8192 785 -> 771).
-#pragma unroll
-        for (int mt = 0; mt < D / 32; mt++) {
-            u16x4 gv[4], sg[4];
-            uint32_t doubt = 0;                // bit 15 - (4 q4 + i)
-#pragma unroll
-            for (int q4 = 0; q4 < 4; q4++)
-                gv[q4] = *reinterpret_cast<const u16x4 *>(gr + mt * 32 + 8 * q4 + 4 * c.h);
-#pragma unroll
-            for (int q4 = 0; q4 < 4; q4++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float g = bf2f(gv[q4][i]);
-                    const float p = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.44269504088896341f));
-                    const bool far = (__float_as_uint(p) << 16) + 0x80100000u >= 0x210000u;
-                    doubt = doubt + doubt + (far && (gv[q4][i] & 0x7fff) <= 0x4180 ? 0u : 1u);
-                    sg[q4][i] = bf_hw(p);
-                }
-            if (__builtin_amdgcn_ballot_w64(doubt != 0)) {
-#pragma unroll
-                for (int e = 0; e < 16; e++)
-                    if (doubt >> (15 - e) & 1u) sg[e >> 2][e & 3] = sig_bf[gv[e >> 2][e & 3]];
-            }
-#pragma unroll
-            for (int q4 = 0; q4 < 4; q4++) {
-                u16x4 out;
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    out[i] = bf_hw(rnd_hw(o[mt][4 * q4 + i]) * bf2f(sg[q4][i]));
-                *reinterpret_cast<u16x4 *>(yr + mt * 32 + 8 * q4 + 4 * c.h) = out;
-            }
-        }
-        // (trace) rnd(o) before the gate, in a loop of its own: a
-        // conditional store inside the loop above would make the compiler
-        // drain the memory counter at every join
-        if (tr_attno) {
-#pragma unroll
-            for (int mt = 0; mt < D / 32; mt++) {
-#pragma unroll
-                for (int q4 = 0; q4 < 4; q4++) {
-                    const int d0 = mt * 32 + 8 * q4 + 4 * c.h;
-                    u16x4 oc;
-#pragma unroll
-                    for (int i = 0; i < 4; i++) oc[i] = f2bf(rndf(o[mt][4 * q4 + i]));
-                    *reinterpret_cast<u16x4 *>(tr_attno + row * D + d0) = oc;
-                }
-            }
-        }
+    if (tk < nt) fa_out(c, o, (size_t)(tb + tk) * nh + head, 0, qg, y, sig_bf, tr_attno);
+}
+
+// ---- k_attn_fa16: tiles of 16 tokens ------------------------------------
+// For calls whose 32-token tiles leave CUs idle (a prompt of 1024 tokens has
+// 64 of them): half the tile, in about two thirds of its time per key tile
+// (T = 1024 96 -> 73 us, 2048 156 -> 117, 4096 292 -> 258; 8192, where all
+// CUs are busy either way, 747 -> 892). Wavefronts g and g + 4, of one SIMD,
+// share query rows: each forms the scores of one 32-key half of a tile, in
+// pass 1 for its own (M, s), joined at the end as the 32-token kernel joins
+// its even and odd steps', and in pass 2 as P, which the two exchange through
+// LDS; each then owns half of d. P.V of a tile runs in the next tile's step,
+// interleaved with forming its P. Every score, sum and P.V chain has the
+// 32-token kernel's order, so a row's bits do not depend on the tile size.
+// V^T has a ring of four blocks: a tile's V is copied a step after its K.
+constexpr int TQ16 = 16;
+constexpr int VRING = 2 * KBUF;                // four V^T blocks (two tiles)
+constexpr int PBUF = VRING + 4 * VHALF;        // P of a tile: [row group][half][lane][32 bytes]
+__global__ __launch_bounds__(64 * NW) void k_attn_fa16(
+    FaSeqs sq, const int32_t *__restrict__ dmeta, const uint16_t *__restrict__ qn_w,
+    const uint16_t *__restrict__ rope,
+    const uint16_t *__restrict__ qg, KvRef kv, int nh, int nkv, float scale,
+    uint16_t *__restrict__ y, const uint16_t *__restrict__ sig_bf, uint16_t *__restrict__ tr_attno) {
+    const int n = sq.n;
+    const int32_t *cu = dmeta ? dmeta : sq.cu;
+    const int32_t *pos0 = dmeta ? dmeta + n + 1 : sq.pos0;
+    const int32_t *toff = dmeta ? dmeta + 2 * n + 1 : sq.toff;
+    const int32_t *hdv = dmeta ? dmeta + 3 * n + 2 : sq.hd;
+    const int ntiles = toff[n];
+    const int g = ntiles - 1 - (int)(blockIdx.x / nkv);
+    const int kvh = blockIdx.x % nkv;
+    // workgroup-uniform (loaded values are not provably so: readfirstlane
+    // keeps them in SGPRs)
+    const int s = __builtin_amdgcn_readfirstlane(seq_of(toff, n, g));
+    const int tb = __builtin_amdgcn_readfirstlane(cu[s] + (g - toff[s]) * TQ16);  // first token
+    const int nt = __builtin_amdgcn_readfirstlane(min(TQ16, cu[s + 1] - tb));
+    const int qpos0 = __builtin_amdgcn_readfirstlane(pos0[s] + (tb - cu[s]));  // its position
+
+    FaCtx c;
+    c.nkeys = qpos0 + nt;
+    c.tid = threadIdx.x;
+    c.lane = c.tid & 63;
+    c.h = c.lane >> 5;
+    c.l32 = c.lane & 31;
+    c.wave = __builtin_amdgcn_readfirstlane(c.tid >> 6);
+    c.kv = kv;
+    c.hd = __builtin_amdgcn_readfirstlane(hdv[s]);
+    c.kvh = kvh;
+    c.nkv = nkv;
+    c.nkt = (c.nkeys + KT - 1) / KT;
+    c.nblk = (c.nkeys + VB - 1) / VB;
+    c.lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_void *)fa_lds);
+    c.c2 = scale * 1.44269504088896341f;
+    const int nkt = c.nkt;
+    // byte offsets of tile u's buffers in fa_lds
+    auto kbuf = [&](int u) { return (u & 1) * KBUF; };
+    auto vbuf = [&](int kt, int half) { return VRING + (2 * (kt & 1) + half) * VHALF; };
+
+    // wavefronts g and g + 4 share the 32 query rows of tokens 4 g .. 4 g + 3
+    const int grp = c.wave & 3, hf = c.wave >> 2;
+    const bool flat = kv.btab == nullptr;
+    const int blk_bytes = nkv * KVB * D * 2;
+    i32x4 kflat = {0, 0, 0, 0}, vflat = {0, 0, 0, 0};
+    if (flat) {
+        const size_t b0 = (size_t)c.hd * kv.bstride * nkv + kvh;   // block 0 of this kv head
+        kflat = dma_rsrc(kv.k + b0 * KVB * D,
+                         (uint32_t)((c.nblk - 1) * blk_bytes + (c.nkeys - KVB * (c.nblk - 1)) * D * 2));
+        vflat = dma_rsrc(kv.v + b0 * D * KVB, (uint32_t)((c.nblk - 1) * blk_bytes + D * KVB * 2));
     }
+    const bool copier = c.wave < 4;
+    int idn[2] = {0, 0}, idc[2] = {0, 0};      // block ids: the next K tile's, this one's
+    auto copy_k = [&](int u, int kt) {
+#pragma unroll
+        for (int half = 0; half < 2; half++) {
+            i32x4 kr = kflat;
+            int off = (2 * kt + half) * blk_bytes;
+            if (!flat) {
+                idc[half] = __builtin_amdgcn_readfirstlane(idn[half]);
+                kr = fa_krsrc(c, kt, half, idc[half]);
+                off = 0;
+            }
+            fa_dma_k(c.lds + kbuf(u), kr, off, c.wave + 4 * half);
+        }
+    };
+    auto copy_v = [&](int kt, const int (&id)[2]) {
+#pragma unroll
+        for (int half = 0; half < 2; half++) {
+            i32x4 vr = vflat;
+            int off = (2 * kt + half) * blk_bytes;
+            if (!flat) {
+                vr = fa_vrsrc(c, kt, half, id[half]);
+                off = 0;
+            }
+            fa_dma_v(c.lds + vbuf(kt, 0), c.lds + vbuf(kt, 1), vr, off, c.wave + 4 * half);
+        }
+    };
+    auto next_ids = [&](int kt) {
+        if (!flat) {
+            idn[0] = fa_block_id(c, fa_block(c, kt, 0));
+            idn[1] = fa_block_id(c, fa_block(c, kt, 1));
+        }
+    };
+    if (copier) {
+        next_ids(0);
+        copy_k(0, 0);
+        next_ids(1 % nkt);
+    }
+    const int tk = grp * 4 + c.l32 / GRP, head = kvh * GRP + c.l32 % GRP;
+    bf16x8 q[D / 16];
+    {
+        const int tq = min(tk, nt - 1);
+        fa_q(c, qg + ((size_t)(tb + tq) * nh + head) * 2 * D, qn_w, rope, qpos0 + tq, q);
+    }
+    FaRow w{qpos0 + tk, -INFINITY, 0.0f, 0.0f};
+    // K tile u of the stream (0 .. 2 nkt - 1) in place; K tile u + 1 and, in pass
+    // 2, V tile u - nkt (read in the next step) on their way
+    auto begin_tile = [&](int u) {
+        fa_publish();
+        if (copier) {
+            const int idv[2] = {idc[0], idc[1]};
+            if (u + 1 < 2 * nkt) {
+                copy_k(u + 1, (u + 1) % nkt);
+                next_ids((u + 2) % nkt);
+            }
+            if (u >= nkt) copy_v(u - nkt, idv);
+        }
+    };
+    const int qminw = qpos0 + 4 * grp;
+    const int hoff = hf * KHALF, hkey = hf * 32;
+#define FA_P1(NEXT, Kn, kj)                                                    \
+    do {                                                                       \
+        const int kj_ = (kj);                                                  \
+        if (kj_ + 31 > qminw) fa_p1_step<NEXT, true>(c, Kn, kj_, q, sc, w);    \
+        else fa_p1_step<NEXT, false>(c, Kn, kj_, q, sc, w);                    \
+    } while (0)
+    // pass 1: this wavefront's 32 keys of each tile
+    begin_tile(0);
+    f32x16 sc = fa_s(c, kbuf(0) + hoff, q);
+    for (int u = 1; u < nkt; u++) {
+        begin_tile(u);
+        FA_P1(true, kbuf(u) + hoff, (u - 1) * KT + hkey);
+    }
+    begin_tile(nkt);
+    FA_P1(false, 0, (nkt - 1) * KT + hkey);
+#undef FA_P1
+    // both halves' (M, s) joined, even 32-key steps first
+    char *pb = fa_lds + PBUF + (grp * 2 * 64 + c.lane) * 32;
+    {
+        *reinterpret_cast<float2 *>(pb + hf * 2048) = make_float2(w.M, w.lsum);
+        __syncthreads();
+        const float2 a = *reinterpret_cast<const float2 *>(pb), b = *reinterpret_cast<const float2 *>(pb + 2048);
+        w.K2 = fa_join(a.x, a.y, b.x, b.y, c.c2);
+    }
+    f32x16 o[D / 64];
+#pragma unroll
+    for (int mt = 0; mt < D / 64; mt++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) o[mt][i] = 0.0f;
+    bf16x8 pm[2], pq[2];                       // P: this wavefront's keys, the partner's
+    // the P.V MFMAs of key tile kt (steps in key order; d tiles 4 hf .. + 3)
+    // around f(i), i = 0 .. 15
+    auto pv = [&](int kt, auto f) {
+        const int vbase = fa_vbase();
+        const bool h1 = hf != 0;
+        bf16x8 b[4];
+#pragma unroll
+        for (int st = 0; st < 2; st++) {
+            b[st] = h1 ? pq[st] : pm[st];
+            b[2 + st] = h1 ? pm[st] : pq[st];
+        }
+        const char *V0 = fa_lds + vbuf(kt, 0) + hf * 4 * 32 * VB * 2;
+        auto va = [&](int jj) {                // operand of MFMA jj: block jj / 8, step jj / 4 % 2, d tile jj % 4
+            return lds16(V0 + (jj >> 3) * VHALF + (vbase ^ (((jj >> 2) & 1) << 5)) + (jj & 3) * 32 * VB * 2);
+        };
+        u16x8 vq[3];
+#pragma unroll
+        for (int i = 0; i < 3; i++) vq[i] = va(i);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int jj = 0; jj < 16; jj++) {
+            const bf16x8 a = __builtin_bit_cast(bf16x8, vq[jj % 3]);
+            if (jj + 3 < 16) vq[jj % 3] = va(jj + 3);
+            o[jj & 3] = mfma32(a, b[jj >> 2], o[jj & 3]);
+            f(jj);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto store_p = [&](const uint32_t (&pw)[8]) {
+#pragma unroll
+        for (int st = 0; st < 2; st++) {
+            const uint4 v = make_uint4(pw[4 * st], pw[4 * st + 1], pw[4 * st + 2], pw[4 * st + 3]);
+            pm[st] = __builtin_bit_cast(bf16x8, v);
+            *reinterpret_cast<uint4 *>(pb + hf * 2048 + st * 16) = v;
+        }
+    };
+    auto load_p = [&] {
+#pragma unroll
+        for (int st = 0; st < 2; st++)
+            pq[st] = *reinterpret_cast<const bf16x8 *>(pb + (hf ^ 1) * 2048 + st * 16);
+    };
+    // P.V of tile kt - 1 while P of tile kt is formed from sc
+    auto step = [&](int kt, auto mask, auto first) {
+        constexpr bool MASK = decltype(mask)::value;
+        const int lim = w.qpos - (kt * KT + hkey) - 8 * (fa_lane() >> 5);
+        uint32_t pw[8], pk = 0;
+        float ep = 0.0f;
+        auto score = [&](int i) {
+            if ((i & 1) == 0) pk = pack2(sc[i], sc[i + 1]);
+            const float r = __uint_as_float((i & 1) ? (pk & 0xffff0000u) : (pk << 16));
+            float ev = __builtin_amdgcn_exp2f(fmaf(r, c.c2, -w.K2));
+            if (MASK) ev = fa_keep(i, lim) ? ev : 0.0f;
+            if (i & 1) pw[i >> 1] = pack2(ep, ev);
+            else ep = ev;
+        };
+        if (decltype(first)::value) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) score(i);
+        } else {
+            pv(kt - 1, score);
+        }
+        store_p(pw);
+    };
+    using yes = std::true_type;
+    using no = std::false_type;
+    sc = fa_s(c, kbuf(nkt) + hoff, q);
+    __syncthreads();                           // every reader of the joined (M, s) is done
+    step(0, yes{}, yes{});
+    const int nmf = (qpos0 + 1) / KT;          // key tiles below it need no mask
+    int kt = 1;
+    for (; kt < nmf; kt++) {
+        begin_tile(nkt + kt);                  // also: P of tile kt - 1 is in place
+        load_p();
+        sc = fa_s(c, kbuf(nkt + kt) + hoff, q);
+        __syncthreads();                       // every reader of that P is done
+        step(kt, no{}, no{});
+    }
+    for (; kt < nkt; kt++) {
+        begin_tile(nkt + kt);
+        load_p();
+        sc = fa_s(c, kbuf(nkt + kt) + hoff, q);
+        __syncthreads();
+        step(kt, yes{}, no{});
+    }
+    fa_publish();                              // the last V tile and P
+    load_p();
+    // the last tile's V keys past nkeys: zero (P is 0 there, but 0 * NaN from
+    // unwritten cache memory would not be)
+    if (c.nkeys % VB != 0) {
+        const int kbase = (nkt - 1) * KT;
+        for (int e = c.tid; e < KT * D; e += 64 * NW) {
+            const int bb = e / (D * VB), rem = e % (D * VB), row = rem / VB, kk = rem % VB;
+            if (kbase + bb * VB + kk >= c.nkeys) {
+                uint16_t *Vn = reinterpret_cast<uint16_t *>(fa_lds + vbuf(nkt - 1, bb));
+                const int cc = (kk >> 3) ^ ((row >> 2) & 3);
+                Vn[row * VB + cc * 8 + (kk & 7)] = 0;
+            }
+        }
+        __syncthreads();
+    }
+    pv(nkt - 1, [](int) {});
+    if (tk < nt)
+        fa_out(c, o, (size_t)(tb + tk) * nh + head, hf * (D / 2), qg, y, sig_bf, tr_attno);
 }
 
 }  // namespace
@@ -799,8 +1083,8 @@ namespace apus {
 // idle: 13 tokens after 8000 positions 497 us. Such a sequence can run
 // through the split-K decode kernels instead, 4 tokens at a time (pieces
 // that share a block-table row): 40 us. The times below are fits of both,
-// in us (FA: 30 + 3.7 per 64-key tile of the longest row, tiles beside
-// each other; decode: 18 + 0.0155 per 64 keys of a piece and kv head).
+// in us (FA: 30 + 3.7 per 64-key tile of the longest row, 32-token tiles
+// beside each other, with 16-token ones about 3/4 of it; decode: 18 + 0.0155 per 64 keys of a piece and kv head).
 struct Short {
     size_t first, last;                // sequences first .. last
     size_t pieces;
@@ -864,6 +1148,38 @@ static int short_run(const Short &r, const ApusHipAttnLayer *L, const int32_t *c
                           y + (size_t)t0 * qd);
 }
 
+// Whether 16-token tiles are the faster ones: the time of the busiest CU with
+// either, from a tile's time alone on a CU (us; fits, kt its 64-key tiles: 28 +
+// 3.7 kt with 32 tokens, 26 + 2.5 kt with 16, the latter a tenth slower where
+// CUs take several), tiles dealt longest first: the longest tile, the mean
+// load, and where a few more tiles than CUs remain, the two that share a CU.
+// (8 prompts of 300 tokens after 300, 304 tiles of 16: 106 us, 160 of 32: 86.)
+template <typename Skip>
+static bool fa_half_tiles(size_t B, const int32_t *cu, const int32_t *pos0, size_t nkv,
+                          const Skip &skip) {
+    const size_t cus = (size_t)cu_count();
+    auto busiest = [&](int tq, double base, double per, double *out) {
+        std::vector<double> t;
+        double sum = 0.0;
+        for (size_t s = 0; s < B; s++) {
+            if (skip(s)) continue;
+            const int n = cu[s + 1] - cu[s];
+            if (t.size() + nkv * (size_t)((n + tq - 1) / tq) > 2 * cus) return false;
+            for (int x = 0; x < n; x += tq) {
+                const double us = base + per * (double)((pos0[s] + std::min(x + tq, n) + KT - 1) / KT);
+                for (size_t h = 0; h < nkv; h++) t.push_back(us);
+                sum += us * (double)nkv;
+            }
+        }
+        std::sort(t.begin(), t.end(), [](double x, double y) { return x > y; });
+        *out = t.empty() ? 0.0 : std::max(t[0], sum / (double)cus);
+        if (t.size() > cus) *out = std::max(*out, t[cus - 1] + t[cus]);
+        return true;
+    };
+    double t16 = 0.0, t32 = 0.0;
+    return busiest(TQ16, 26.0, 2.5, &t16) && busiest(TQ, 28.0, 3.7, &t32) && 1.1 * t16 < t32;
+}
+
 int attn_prefill_kv(const ApusHipAttnLayer *L, size_t B, const int32_t *cu, const int32_t *pos0,
                     const int32_t *rows, const uint16_t *qg, const uint16_t *k,
                     const uint16_t *v, const KvRef &kv, uint16_t *y) {
@@ -893,11 +1209,14 @@ int attn_prefill_kv(const ApusHipAttnLayer *L, size_t B, const int32_t *cu, cons
     for (size_t s = 0; s < B; s++) {
         const int32_t ns = cu[s + 1] - cu[s];
         max_pos = std::max(max_pos, (size_t)pos0[s] + (size_t)ns);
-        mtoff[s + 1] = mtoff[s] + (is_short(s) ? 0 : (ns + TQ - 1) / TQ);
         mhd[s] = rows ? rows[s] : (int32_t)s;
     }
     memcpy(mcu, cu, (B + 1) * 4);
     memcpy(mpos, pos0, B * 4);
+    const bool half = fa_half_tiles(B, cu, pos0, L->nkv, is_short);
+    const int32_t tq = half ? TQ16 : TQ;
+    for (size_t s = 0; s < B; s++)
+        mtoff[s + 1] = mtoff[s] + (is_short(s) ? 0 : (cu[s + 1] - cu[s] + tq - 1) / tq);
     const size_t ntiles = (size_t)mtoff[B];
     for (const Short &r : shorts)
         if (int e = short_run(r, L, cu, pos0, rows, qg, k, v, kv, y)) return e;
@@ -933,7 +1252,7 @@ int attn_prefill_kv(const ApusHipAttnLayer *L, size_t B, const int32_t *cu, cons
     const ActTables *tabs = act_tables();
     if (!tabs) return kErrHip;
     APUS_TIMED("k_attn_fa",
-               k_attn_fa<<<(unsigned)(ntiles * L->nkv), 64 * NW, 0, stream()>>>(
+               (half ? k_attn_fa16 : k_attn_fa)<<<(unsigned)(ntiles * L->nkv), 64 * NW, 0, stream()>>>(
                    fs, fdm, L->qn_w, rope, qg, kv, (int)L->nh, (int)L->nkv, scale, y, tabs->sig_bf,
                    attn_trace() ? attn_trace()->attno : nullptr));
     APUS_LAUNCHED("k_attn_fa");

@@ -153,6 +153,37 @@ def test_prefill_short_continuations(hip, orc, lens, pos0):
     _run(hip, orc, np.random.default_rng(len(lens)), cu, pos0, 4032, tag="short")
 
 
+@pytest.mark.parametrize("lens,pos0", [
+    ([1], [0]), ([15], [0]), ([16], [47]), ([17], [31]), ([33], [95]),   # tile and key-tile edges
+    ([63], [1]), ([130], [300]), ([1000], [0])])
+def test_prefill_tile_sizes_agree(hip, orc, lens, pos0):
+    """A call alone runs in 16-token tiles; beside a sequence long enough to
+    fill the chip it runs in 32-token ones. Against the oracle, and the same
+    bits and cache either way."""
+    import torch
+    dims = synth.ATTN_DIMS
+    nh, nkv, d, rot, theta = dims
+    n, p, fill, max_seq = lens[0], pos0[0], 4700, 4704
+    rng = np.random.default_rng(n)
+    if n <= 130:
+        _run(hip, orc, rng, [0, n], pos0, 448, tag="tile")
+    layer = hip.attn_layer(dims, {k: _td(torch, v) for k, v in synth.attn_weights(rng).items()})
+    t = {k: _td(torch, v) for k, v in synth.attn_tokens(rng, n + fill).items()}
+    dk = torch.zeros((2, nkv, max_seq, d), dtype=torch.int16, device="cuda")
+    dv = torch.zeros((2, nkv, max_seq // 32, d, 32), dtype=torch.int16, device="cuda")
+    hip.attn_cache_pack(_td(torch, synth.normal_bf16(rng, (p + 1, nkv, d))),
+                        _td(torch, synth.normal_bf16(rng, (p + 1, nkv, d))), p + 1, nkv, d,
+                        dk[0], dv[0], max_seq)
+    dk1, dv1 = dk[:1].clone(), dv[:1].clone()
+    y = torch.empty((n + fill, nh * d), dtype=torch.int16, device="cuda")
+    hip.attn_prefill(layer, [0, n, n + fill], [p, 0], t["qg"], t["k"], t["v"], dk, dv, max_seq, y)
+    y1 = torch.empty((n, nh * d), dtype=torch.int16, device="cuda")
+    hip.attn_prefill(layer, [0, n], [p], t["qg"][:n], t["k"][:n], t["v"][:n], dk1, dv1, max_seq, y1)
+    torch.cuda.synchronize()
+    assert torch.equal(dk[0], dk1[0]) and torch.equal(dv[0], dv1[0])
+    assert torch.equal(y[:n], y1)
+
+
 def test_prefill_long(hip, orc):
     """One 2048-token causal prefill from position 0 (config 3's shape at a
     quarter of its length)."""
