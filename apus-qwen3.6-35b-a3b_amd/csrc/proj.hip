@@ -4,7 +4,7 @@
 // reference's apus_bf16_gemv_hot / apus_bf16_gemm_hot and the
 // ApusBackendHooks bf16_gemv / bf16_gemm slots (c/backend_metal.h:68-75).
 //
-// Two kernels:
+// The kernels:
 //   k_gemm_seq   one lane per output, the k sum in the reference's order
 //                (ascending, one rounding per multiply and per add: the
 //                scalar anchor c/bf16.h:285-293, which the reference's
@@ -13,6 +13,9 @@
 //                aside: see k_gemm_seq). The weight row is read 16 bytes
 //                at a time, 16 to 32 pieces ahead of the add chain; the x row
 //                is staged in LDS once per wavefront.
+//   k_gemm_seq64 the same chains (K a multiple of 64), the weights streamed
+//                and widened into LDS by wavefronts of their own for up to
+//                four rows at a time.
 //   k_gemm_tile  the 32x32x16 bf16 MFMA with fp32 accumulation, for every
 //                row count: a workgroup computes a (BO outputs x BM rows)
 //                tile, its operands copied global -> LDS by buffer_load ...
@@ -23,8 +26,8 @@
 //                with enough tiles to fill the chip. The tile shape (and
 //                with it the kernel) is the one with the least estimated
 //                time; every shape accumulates an element's k16 steps in
-//                the same order. They sum in their own order: the
-//                tolerance class of the attention kernels (|c - r| <=
+//                the same order. The MFMA kernels sum in their own order:
+//                the tolerance class of the attention kernels (|c - r| <=
 //                2e-3 (|r| + esc), esc = sum_k |w x|).
 // Host-pointer drop-ins keep device copies of the weights keyed by their
 // host address, as the reference's Metal backend keys weights by stable
@@ -513,6 +516,12 @@ __global__ __launch_bounds__(64 * WO * WM) void k_gemm_tile(GemmSegs sg,
 // The stores of a tile go through LDS as whole rows (what a call takes
 // besides its k steps: 23 -> 7 us). 4096 x 12352 x 2048: 236 -> 201 us (1.03
 // PFLOP/s).
+// The ring holds ST stages. Three where a CU has LDS for them beside the
+// fewer products of a small tile, which a copy of one stage outlasts
+// (325 x 12352 x 2048, 194 workgroups of 128 x 192: two stages 29.3 us, three
+// 25.6; four, at 128 x 128, no further gain), two for 256-wide tiles, and
+// for 128 x 128 where two workgroups share a CU (640 x 12352: 38 us, with
+// three stages one after the other 43).
 constexpr int kWideK = 64;                // k per stage
 
 // 16 (4) bytes per lane from a 64-bit address to LDS byte lds + 16 (4) *
@@ -539,7 +548,7 @@ __device__ __forceinline__ void dma4_g(const char *p, uint32_t lds) {
 // 16-byte chunk c of row r at slot c ^ (r % 8), so that the 8 rows of one
 // LDS read phase hit 8 distinct slots. K is a multiple of 32: an odd last
 // half stage has no second half to read, so its copies repeat the first.
-template <int TO, int TMM>
+template <int TO, int TMM, int ST>
 __device__ __forceinline__ void gemm_wide(char *sm, const GemmSegs &sg, const uint16_t *x, int M,
                                           int K, int o0, int m0, int sw, int iw, int ix) {
     constexpr int NW = 4, BO = 64 * TO, BM = 64 * TMM;
@@ -590,10 +599,10 @@ __device__ __forceinline__ void gemm_wide(char *sm, const GemmSegs &sg, const ui
         const bool px = e >= nw && e < nw + nx;
         const int o = min(o0 + iw * nw + (e < nw ? e : 0), O - 1), si = seg_of(sg, o);
         const int row = px ? min(m0 + ix * nx + e - nw, M - 1) : o - sg.row0[si];
-        pf = (const char *)((px ? x : sg.w[si]) + (size_t)row * K) + min(2, nk - 1) * 128;
+        pf = (const char *)((px ? x : sg.w[si]) + (size_t)row * K) + min(ST, nk - 1) * 128;
     }
-    auto prefetch = [&](int st) {            // stages 2, 3, ... in turn
-        dma4_g(pf, lds0 + 2 * SB + wave * 256);
+    auto prefetch = [&](int st) {            // stages ST, ST + 1, ... in turn
+        dma4_g(pf, lds0 + ST * SB + wave * 256);
         pf += st + 1 < nk ? 128 : 0;
     };
     f32x16 acc[TO][TMM];
@@ -640,14 +649,17 @@ __device__ __forceinline__ void gemm_wide(char *sm, const GemmSegs &sg, const ui
         }
     };
     Frag f0, f1;
-    // stages 0 and 1 in flight; stage 0 published
-    const int adv0 = advance(0), adv1 = advance(1);
+    // stages 0 .. ST - 1 in flight; stage 0 published
 #pragma unroll
-    for (int i = 0; i < PPW; i++) copy(i, 0, adv0, -1);
+    for (int st = 0; st < ST; st++) {
+        const int adv = advance(st);
 #pragma unroll
-    for (int i = 0; i < PPW; i++) copy(i, SB, adv1, (1 - nk) >> 31);
-    prefetch(2);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PPW + 1) : "memory");
+        for (int i = 0; i < PPW; i++) copy(i, st * SB, adv, (st - nk) >> 31);
+    }
+    prefetch(ST);
+    // (the counts take every copy after the awaited ones as a live one)
+    if (nk >= ST) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PPW * (ST - 1) + 1) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < NR; j++) rd1(0, 0, j, f0);
@@ -658,13 +670,15 @@ __device__ __forceinline__ void gemm_wide(char *sm, const GemmSegs &sg, const ui
         step(f0, f1, yes{}, slot, 3, no{}, 0, 0, 0);
         // every operand of this stage has been read, by this wavefront (it
         // waited for f1) and after the barrier by all, and the next stage has
-        // landed (its copies are older than the last prefetch): stage
-        // kt + 2 goes into this stage's slot
-        asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
+        // landed (its copies are older than those of ST - 2 stages and the
+        // last prefetch): stage kt + ST goes into this stage's slot
+        if (kt + ST <= nk) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PPW * (ST - 2) + 1) : "memory");
+        else asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
         __syncthreads();
-        step(f1, f0, yes{}, slot ^ SB, 0, yes{}, slot, advance(kt + 2), (kt + 2 - nk) >> 31);
-        prefetch(kt + 3);
-        slot ^= SB;
+        const uint32_t next = slot + SB == ST * SB ? 0 : slot + SB;
+        step(f1, f0, yes{}, next, 0, yes{}, slot, advance(kt + ST), (kt + ST - nk) >> 31);
+        prefetch(kt + ST + 1);
+        slot = next;
     }
     // the last stage; an odd K's second half is zeros
     auto mask = [&](Frag &f) {
@@ -730,11 +744,11 @@ __device__ __forceinline__ void gemm_wide(char *sm, const GemmSegs &sg, const ui
 template <int TO>
 __host__ __device__ inline bool wide_narrow(int O) { return TO == 4 && O % 256 > 0 && O % 256 <= 64 && O > 256; }
 
-template <int TO, int TMM>
-__global__ __launch_bounds__(256, TO * TMM <= 8 ? 2 : 1) void k_gemm_wide(
+template <int TO, int TMM, int ST>
+__global__ __launch_bounds__(256, TO * TMM <= 8 && ST == 2 ? 2 : 1) void k_gemm_wide(
     GemmSegs sg, const uint16_t *__restrict__ x, int M, int K) {
     constexpr int BO = 64 * TO, BM = 64 * TMM;
-    __shared__ __attribute__((aligned(16))) char sm[2 * (BO + BM) * 128 + 1024];
+    __shared__ __attribute__((aligned(16))) char sm[ST * (BO + BM) * 128 + 1024];
     const int O = sg.row0[sg.n];
     const bool narrow = wide_narrow<TO>(O);
     const int nbo = narrow ? O / BO : (O + BO - 1) / BO, nbm = (M + BM - 1) / BM;
@@ -742,13 +756,13 @@ __global__ __launch_bounds__(256, TO * TMM <= 8 ? 2 : 1) void k_gemm_wide(
     // the workgroups of this one's XCD that share its tiles (tile_of)
     const int sw = min(nbm, 8);
     if (TO == 4 && (int)blockIdx.x >= n) {
-        gemm_wide<1, TMM>(sm, sg, x, M, K, nbo * BO, ((int)blockIdx.x - n) * BM, 1, 0, 0);
+        gemm_wide<1, TMM, ST>(sm, sg, x, M, K, nbo * BO, ((int)blockIdx.x - n) * BM, 1, 0, 0);
         return;
     }
     int ob, mb;
     tile_of(blockIdx.x, nbo, nbm, ob, mb);
     if (ob >= nbo) return;                      // (the grid is a multiple of 8)
-    gemm_wide<TO, TMM>(sm, sg, x, M, K, ob * BO, mb * BM, sw, mb % sw, ob % (32 / sw));
+    gemm_wide<TO, TMM, ST>(sm, sg, x, M, K, ob * BO, mb * BM, sw, mb % sw, ob % (32 / sw));
 }
 
 // y = rnd(sum over the splits of part, in split order), scattered to the
@@ -795,13 +809,13 @@ int launch_tile(const GemmSegs &sg, const uint16_t *x, int M, int K, const char 
     return kOk;
 }
 
-template <int TO, int TMM>
+template <int TO, int TMM, int ST>
 int launch_wide(const GemmSegs &sg, const uint16_t *x, int M, int K, const char *name) {
     constexpr int BO = 64 * TO, BM = 64 * TMM;
     const int O = sg.row0[sg.n], nbm = (M + BM - 1) / BM;
     const bool narrow = wide_narrow<TO>(O);
     const unsigned grid = (unsigned)(tile_grid(narrow ? O / BO : (O + BO - 1) / BO, nbm) + (narrow ? nbm : 0));
-    APUS_TIMED(name, k_gemm_wide<TO, TMM><<<grid, 256, 0, stream()>>>(sg, x, M, K));
+    APUS_TIMED(name, k_gemm_wide<TO, TMM, ST><<<grid, 256, 0, stream()>>>(sg, x, M, K));
     return launch_check(name);
 }
 
@@ -818,18 +832,19 @@ struct TileShape {
     bool split;                             // has a K-split form
     int (*run)(const GemmSegs &, const uint16_t *, int, int, const char *, int);
 };
-template <int TO, int TMM>
+template <int TO, int TMM, int ST>
 int run_wide(const GemmSegs &sg, const uint16_t *x, int M, int K, const char *nm, int) {
-    return launch_wide<TO, TMM>(sg, x, M, K, nm);
+    return launch_wide<TO, TMM, ST>(sg, x, M, K, nm);
 }
 const TileShape kTileShapes[] = {
     {64, 64, 12.7f, 0.0f, 20.5f, true, launch_tile<2, 1, 1, 2>},
     {128, 64, 15.5f, 0.0f, 33.0f, true, launch_tile<2, 2, 2, 1>},
     {128, 128, 24.0f, 6.5f, 50.0f, true, launch_tile<2, 4, 2, 1>},
-    {128, 128, 27.0f, 2.0f, 41.5f, false, run_wide<2, 2>},
-    {128, 192, 31.0f, 4.0f, 64.6f, false, run_wide<2, 3>},
-    {256, 192, 49.0f, 10.0f, 97.0f, false, run_wide<4, 3>},
-    {256, 256, 62.0f, 12.0f, 124.0f, false, run_wide<4, 4>},
+    {128, 128, 27.0f, 2.0f, 41.5f, false, run_wide<2, 2, 2>},
+    {128, 128, 22.5f, 3.0f, 47.0f, false, run_wide<2, 2, 3>},
+    {128, 192, 27.5f, 3.0f, 62.0f, false, run_wide<2, 3, 3>},
+    {256, 192, 49.0f, 10.0f, 97.0f, false, run_wide<4, 3, 2>},
+    {256, 256, 62.0f, 12.0f, 124.0f, false, run_wide<4, 4, 2>},
 };
 
 }  // namespace

@@ -135,7 +135,8 @@ def test_gemm_mfma_tolerance(hip, orc, M, O, K):
 # stage, of half a stage and with an odd half stage.
 @pytest.mark.parametrize("M,O,K", [(4096, 576, 64), (2300, 4160, 2048), (1025, 12352, 96),
                                    (700, 12353, 32), (1537, 8200, 160), (769, 12356, 2080),
-                                   (385, 12320, 64), (129, 12352, 192), (3001, 2049, 1056)])
+                                   (385, 12320, 64), (129, 12352, 192), (3001, 2049, 1056),
+                                   (200, 12352, 32), (325, 12352, 128), (300, 12345, 288)])
 def test_gemm_mfma_tile_shapes_agree(hip, M, O, K):
     import torch
     print(f"[proj] shapes M={M} O={O} K={K}", flush=True)
