@@ -1101,8 +1101,9 @@ static bool short_seq(int64_t n, int64_t pos0, size_t nkv, double *groups) {
 }
 // The runs of short sequences to take out of the flash kernel's grid: all or
 // none, if that saves more than it costs. Bounds: one call's by-value
-// metadata, and 100 MB of scores in library scratch.
+// metadata, and what the scratch below holds.
 constexpr double kShortGroups = 24576.0;
+constexpr size_t kShortPairs = 512;    // (piece, kv head) pairs
 static std::vector<Short> short_runs(size_t B, const int32_t *cu, const int32_t *pos0, size_t nkv) {
     std::vector<Short> runs;
     double groups = 0.0, t_short = 0.0, t_rest = 0.0, sum = 0.0;
@@ -1124,10 +1125,38 @@ static std::vector<Short> short_runs(size_t B, const int32_t *cu, const int32_t 
         }
     }
     t_rest = std::max(t_rest, sum / (double)cu_count());
-    if (pieces > (size_t)kAttnInlineSeqs || groups > kShortGroups ||
+    if (pieces > (size_t)kAttnInlineSeqs || pieces * nkv > kShortPairs || groups > kShortGroups ||
         18.0 * (double)runs.size() + 0.0155 * groups > 0.8 * (t_short - t_rest))
         runs.clear();
     return runs;
+}
+// Scratch for the largest such runs, in slots of their own and allocated once:
+// a prefill then neither moves a buffer that a captured decode holds nor
+// shares one with a decode on another stream. Where it cannot be had (memory;
+// an allocation during capture) the flash kernel runs instead. Calls on two
+// streams take turns: the first on another stream than the last waits.
+static bool short_scratch() {
+    constexpr size_t kRowsP = 4 * GRP;                     // rows of a pair
+    const size_t cus = (size_t)cu_count();                 // at most 16 runs of scores, 3 of P.V a CU
+    const size_t need[4] = {kShortPairs * kRowsP * D * 2, (size_t)kShortGroups * 64 * kRowsP * 2,
+                            (16 * cus + kShortPairs) * kRowsP * 8,
+                            (3 * cus + kShortPairs) * kRowsP * D * 4};
+    static hipStream_t last = nullptr;
+    bool held = true;
+    for (int i = 0; i < 4; i++) held = held && scratch_held(kScratchShortQ + i, need[i]);
+    if (held && last == stream()) return true;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream(), &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return false;
+    }
+    for (int i = 0; i < 4; i++) held = scratch(kScratchShortQ + i, need[i]) != nullptr && (i == 0 || held);
+    if (!held || (last != stream() && hipDeviceSynchronize() != hipSuccess)) {
+        (void)hipGetLastError();
+        return false;
+    }
+    last = stream();
+    return true;
 }
 // The sequences of r as pieces of at most 4 tokens through the decode path.
 // (Every piece's k and v rows are in the cache before any piece's scores.)
@@ -1145,7 +1174,7 @@ static int short_run(const Short &r, const ApusHipAttnLayer *L, const int32_t *c
     const size_t qd = L->nh * D, kd = L->nkv * D;
     return attn_decode_kv(L, ppos.size(), pcu.data(), ppos.data(), prow.data(),
                           qg + (size_t)t0 * 2 * qd, k + (size_t)t0 * kd, v + (size_t)t0 * kd, kv,
-                          y + (size_t)t0 * qd);
+                          y + (size_t)t0 * qd, kScratchShortQ);
 }
 
 // Whether 16-token tiles are the faster ones: the time of the busiest CU with
@@ -1197,6 +1226,7 @@ int attn_prefill_kv(const ApusHipAttnLayer *L, size_t B, const int32_t *cu, cons
     // (a trace's buffers are indexed by the call's tokens: not in pieces)
     std::vector<Short> shorts;
     if (!attn_trace()) shorts = short_runs(B, cu, pos0, L->nkv);
+    if (!shorts.empty() && !short_scratch()) shorts.clear();
     auto is_short = [&](size_t s) {
         for (const Short &r : shorts)
             if (s >= r.first && s <= r.last) return true;

@@ -184,6 +184,38 @@ def test_prefill_tile_sizes_agree(hip, orc, lens, pos0):
     assert torch.equal(y[:n], y1)
 
 
+def test_prefill_short_on_two_streams(hip):
+    """Short continuations keep their scratch in place and take turns where
+    the stream changes: the same bits on either stream, back to back."""
+    import torch
+    dims = synth.ATTN_DIMS
+    nh, nkv, d, rot, theta = dims
+    rng = np.random.default_rng(8)
+    n, p, max_seq = 13, 3000, 3040
+    layer = hip.attn_layer(dims, {k: _td(torch, v) for k, v in synth.attn_weights(rng).items()})
+    t = {k: _td(torch, v) for k, v in synth.attn_tokens(rng, n).items()}
+    kc, vc = (_td(torch, synth.normal_bf16(rng, (p, nkv, d))) for _ in range(2))
+    ys, keep = [], []
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    try:
+        for i in range(4):
+            hip.set_stream(streams[i % 2].cuda_stream)
+            with torch.cuda.stream(streams[i % 2]):
+                dk = torch.zeros((1, nkv, max_seq, d), dtype=torch.int16, device="cuda")
+                dv = torch.zeros((1, nkv, max_seq // 32, d, 32), dtype=torch.int16, device="cuda")
+                y = torch.zeros((n, nh * d), dtype=torch.int16, device="cuda")
+                hip.attn_cache_pack(kc, vc, p, nkv, d, dk[0], dv[0], max_seq)
+                hip.attn_prefill(layer, [0, n], [p], t["qg"], t["k"], t["v"], dk, dv, max_seq, y)
+            ys.append(y)
+            keep += [dk, dv]
+        torch.cuda.synchronize()
+    finally:
+        hip.set_stream(None)
+    for y in ys[1:]:
+        assert torch.equal(ys[0], y)
+
+
 def test_prefill_long(hip, orc):
     """One 2048-token causal prefill from position 0 (config 3's shape at a
     quarter of its length)."""
