@@ -145,8 +145,6 @@ int current_device() { return g_device; }
 hipStream_t stream() { return g_stream; }
 void set_stream(hipStream_t s) { g_stream = s; }
 
-bool scratch_held(int slot, size_t bytes) { return g_scratch[slot].n >= bytes; }
-
 void *scratch(int slot, size_t bytes) {
     Buf &b = g_scratch[slot];
     if (bytes == 0) bytes = 1;

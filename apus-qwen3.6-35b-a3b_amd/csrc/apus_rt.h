@@ -59,15 +59,11 @@ enum ScratchSlot { kScratchIn = 0, kScratchIn2, kScratchIn3, kScratchIn4,
                    // batched attention mixer intermediates
                    kScratchAttnQ, kScratchAttnA, kScratchAttnStat,
                    kScratchAttnPart,
-                   // the same four for attention prefill's short continuations
-                   kScratchShortQ, kScratchShortA, kScratchShortStat,
-                   kScratchShortPart,
                    // layer entry points: projection outputs, mixer output
                    kScratchLayerA, kScratchLayerB, kScratchLayerC, kScratchLayerD,
                    kScratchLayerY,
                    kScratchSlots };
 void *scratch(int slot, size_t bytes);
-bool scratch_held(int slot, size_t bytes);   // scratch() would not allocate
 
 // Device RoPE table for (rot, theta): [npos][rot] bf16 codes, per
 // position cos for pairs 0..rot/2-1 then sin. Computed on the host with

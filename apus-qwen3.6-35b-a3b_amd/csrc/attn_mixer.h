@@ -96,10 +96,9 @@ int kv_paged_ref(const ApusHipKvCache *c, size_t B, const int32_t *rows, const i
 int attn_prefill_kv(const ApusHipAttnLayer *L, size_t B, const int32_t *cu, const int32_t *pos0,
                     const int32_t *rows, const uint16_t *qg, const uint16_t *k,
                     const uint16_t *v, const KvRef &kv, uint16_t *y);
-// Decode on a cache given as a KvRef (flat or paged), with its intermediates
-// in the four scratch slots from `slots` (in kScratchAttnQ's order).
+// Decode on a cache given as a KvRef (flat or paged).
 int attn_decode_kv(const ApusHipAttnLayer *L, size_t B, const int32_t *cu, const int32_t *pos0,
                    const int32_t *rows, const uint16_t *qg, const uint16_t *k,
-                   const uint16_t *v, const KvRef &kv, uint16_t *y, int slots = kScratchAttnQ);
+                   const uint16_t *v, const KvRef &kv, uint16_t *y);
 
 }  // namespace apus

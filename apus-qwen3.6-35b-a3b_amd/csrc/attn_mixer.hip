@@ -1315,7 +1315,7 @@ int attn_max_vblocks(size_t B, const int32_t *cu, const int32_t *pos0) {
 
 int attn_decode_kv(const ApusHipAttnLayer *L, size_t B, const int32_t *cu, const int32_t *pos0,
                    const int32_t *rows, const uint16_t *qg, const uint16_t *k,
-                   const uint16_t *v, const KvRef &kv, uint16_t *y, int slots) {
+                   const uint16_t *v, const KvRef &kv, uint16_t *y) {
     if (int r = attn_check_layer(L)) return r;
     if (B == 0) return kOk;
     AttnSeqs sq;
@@ -1333,10 +1333,10 @@ int attn_decode_kv(const ApusHipAttnLayer *L, size_t B, const int32_t *cu, const
     const size_t max_cap = ceil64(max_pos);
     const size_t total = nkv * keys;
     const size_t nruns1 = (total + sq.T1 - 1) / sq.T1, nruns2 = (total + sq.T2 - 1) / sq.T2;
-    uint16_t *qn = (uint16_t *)scratch(slots, Ttot * L->nh * D * 2);
-    uint16_t *As = (uint16_t *)scratch(slots + 1, total * kRows * 2);
-    float2 *st = (float2 *)scratch(slots + 2, (nruns1 + B * nkv) * kRows * 8);
-    float *Op = (float *)scratch(slots + 3, (nruns2 + B * nkv) * kRows * D * 4);
+    uint16_t *qn = (uint16_t *)scratch(kScratchAttnQ, Ttot * L->nh * D * 2);
+    uint16_t *As = (uint16_t *)scratch(kScratchAttnA, total * kRows * 2);
+    float2 *st = (float2 *)scratch(kScratchAttnStat, (nruns1 + B * nkv) * kRows * 8);
+    float *Op = (float *)scratch(kScratchAttnPart, (nruns2 + B * nkv) * kRows * D * 4);
     if (!qn || !As || !st || !Op) return kErrHip;
     if (int r = attn_prep(L, sq, dmeta, Ttot, max_pos, attn_max_vblocks(B, cu, pos0), qg, k, v,
                           kv, qn))

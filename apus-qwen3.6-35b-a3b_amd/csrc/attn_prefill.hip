@@ -1077,121 +1077,18 @@ __global__ __launch_bounds__(64 * NW) void k_attn_fa16(
 
 namespace apus {
 
-// Short continuations of long prefixes (the next turn of a long chat). A
-// query tile of 32 tokens walks all its keys on one CU, twice, so a few new
-// tokens after a long prefix take as long as a full tile while most CUs
-// idle: 13 tokens after 8000 positions 497 us. Such a sequence can run
-// through the split-K decode kernels instead, 4 tokens at a time (pieces
-// that share a block-table row): 40 us. The times below are fits of both,
-// in us (FA: 30 + 3.7 per 64-key tile of the longest row, 32-token tiles
-// beside each other, with 16-token ones about 3/4 of it; decode: 18 + 0.0155 per 64 keys of a piece and kv head).
-struct Short {
-    size_t first, last;                // sequences first .. last
-    size_t pieces;
-    double groups;                     // 64-key groups over pieces and kv heads
-};
-static double fa_us(int64_t keys) { return 30.0 + 3.7 * (double)((keys + KT - 1) / KT); }
-// A sequence is short by its own sizes alone (so it goes the same way in
-// any batch that is not much larger): a prefix of at least 512 positions
-// and four times the new tokens, and less than half the time.
-static bool short_seq(int64_t n, int64_t pos0, size_t nkv, double *groups) {
-    if (n < 1 || pos0 < 512 || pos0 < 4 * n) return false;
-    *groups = (double)((n + 3) / 4) * (double)nkv * (double)((pos0 + n + 63) / 64);
-    return 18.0 + 0.0155 * *groups < 0.5 * fa_us(pos0 + n);
-}
-// The runs of short sequences to take out of the flash kernel's grid: all or
-// none, if that saves more than it costs. Bounds: one call's by-value
-// metadata, and what the scratch below holds.
-constexpr double kShortGroups = 24576.0;
-constexpr size_t kShortPairs = 512;    // (piece, kv head) pairs
-static std::vector<Short> short_runs(size_t B, const int32_t *cu, const int32_t *pos0, size_t nkv) {
-    std::vector<Short> runs;
-    double groups = 0.0, t_short = 0.0, t_rest = 0.0, sum = 0.0;
-    size_t pieces = 0;
-    for (size_t s = 0; s < B; s++) {
-        const int64_t n = cu[s + 1] - cu[s];
-        double g = 0.0;
-        if (short_seq(n, pos0[s], nkv, &g)) {
-            if (runs.empty() || runs.back().last + 1 != s) runs.push_back(Short{s, s, 0, 0.0});
-            runs.back().last = s;
-            runs.back().pieces += (size_t)(n + 3) / 4;
-            runs.back().groups += g;
-            groups += g;
-            pieces += (size_t)(n + 3) / 4;
-            t_short = std::max(t_short, fa_us(pos0[s] + n));
-        } else if (n > 0) {
-            t_rest = std::max(t_rest, fa_us(pos0[s] + n));
-            sum += (double)nkv * (double)((n + TQ - 1) / TQ) * (fa_us(pos0[s] + n / 2) - 20.0);
-        }
-    }
-    t_rest = std::max(t_rest, sum / (double)cu_count());
-    if (pieces > (size_t)kAttnInlineSeqs || pieces * nkv > kShortPairs || groups > kShortGroups ||
-        18.0 * (double)runs.size() + 0.0155 * groups > 0.8 * (t_short - t_rest))
-        runs.clear();
-    return runs;
-}
-// Scratch for the largest such runs, in slots of their own and allocated once:
-// a prefill then neither moves a buffer that a captured decode holds nor
-// shares one with a decode on another stream. Where it cannot be had (memory;
-// an allocation during capture) the flash kernel runs instead. Calls on two
-// streams take turns: the first on another stream than the last waits.
-static bool short_scratch() {
-    constexpr size_t kRowsP = 4 * GRP;                     // rows of a pair
-    const size_t cus = (size_t)cu_count();                 // at most 16 runs of scores, 3 of P.V a CU
-    const size_t need[4] = {kShortPairs * kRowsP * D * 2, (size_t)kShortGroups * 64 * kRowsP * 2,
-                            (16 * cus + kShortPairs) * kRowsP * 8,
-                            (3 * cus + kShortPairs) * kRowsP * D * 4};
-    static hipStream_t last = nullptr;
-    bool held = true;
-    for (int i = 0; i < 4; i++) held = held && scratch_held(kScratchShortQ + i, need[i]);
-    if (held && last == stream()) return true;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream(), &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        return false;
-    }
-    for (int i = 0; i < 4; i++) held = scratch(kScratchShortQ + i, need[i]) != nullptr && (i == 0 || held);
-    if (!held || (last != stream() && hipDeviceSynchronize() != hipSuccess)) {
-        (void)hipGetLastError();
-        return false;
-    }
-    last = stream();
-    return true;
-}
-// The sequences of r as pieces of at most 4 tokens through the decode path.
-// (Every piece's k and v rows are in the cache before any piece's scores.)
-static int short_run(const Short &r, const ApusHipAttnLayer *L, const int32_t *cu,
-                     const int32_t *pos0, const int32_t *rows, const uint16_t *qg,
-                     const uint16_t *k, const uint16_t *v, const KvRef &kv, uint16_t *y) {
-    std::vector<int32_t> pcu{0}, ppos, prow;
-    const int32_t t0 = cu[r.first];
-    for (size_t s = r.first; s <= r.last; s++)
-        for (int32_t t = cu[s]; t < cu[s + 1]; t += 4) {
-            pcu.push_back(std::min(t + 4, cu[s + 1]) - t0);
-            ppos.push_back(pos0[s] + (t - cu[s]));
-            prow.push_back(rows ? rows[s] : (int32_t)s);
-        }
-    const size_t qd = L->nh * D, kd = L->nkv * D;
-    return attn_decode_kv(L, ppos.size(), pcu.data(), ppos.data(), prow.data(),
-                          qg + (size_t)t0 * 2 * qd, k + (size_t)t0 * kd, v + (size_t)t0 * kd, kv,
-                          y + (size_t)t0 * qd, kScratchShortQ);
-}
-
 // Whether 16-token tiles are the faster ones: the time of the busiest CU with
 // either, from a tile's time alone on a CU (us; fits, kt its 64-key tiles: 28 +
 // 3.7 kt with 32 tokens, 26 + 2.5 kt with 16, the latter a tenth slower where
 // CUs take several), tiles dealt longest first: the longest tile, the mean
 // load, and where a few more tiles than CUs remain, the two that share a CU.
 // (8 prompts of 300 tokens after 300, 304 tiles of 16: 106 us, 160 of 32: 86.)
-template <typename Skip>
-static bool fa_half_tiles(size_t B, const int32_t *cu, const int32_t *pos0, size_t nkv,
-                          const Skip &skip) {
+static bool fa_half_tiles(size_t B, const int32_t *cu, const int32_t *pos0, size_t nkv) {
     const size_t cus = (size_t)cu_count();
     auto busiest = [&](int tq, double base, double per, double *out) {
         std::vector<double> t;
         double sum = 0.0;
         for (size_t s = 0; s < B; s++) {
-            if (skip(s)) continue;
             const int n = cu[s + 1] - cu[s];
             if (t.size() + nkv * (size_t)((n + tq - 1) / tq) > 2 * cus) return false;
             for (int x = 0; x < n; x += tq) {
@@ -1223,15 +1120,6 @@ int attn_prefill_kv(const ApusHipAttnLayer *L, size_t B, const int32_t *cu, cons
         return r;
     const size_t Ttot = (size_t)cu[B];
     if (Ttot == 0) return kOk;
-    // (a trace's buffers are indexed by the call's tokens: not in pieces)
-    std::vector<Short> shorts;
-    if (!attn_trace()) shorts = short_runs(B, cu, pos0, L->nkv);
-    if (!shorts.empty() && !short_scratch()) shorts.clear();
-    auto is_short = [&](size_t s) {
-        for (const Short &r : shorts)
-            if (s >= r.first && s <= r.last) return true;
-        return false;
-    };
     size_t max_pos = 0;
     std::vector<int32_t> meta(4 * B + 2);
     int32_t *mcu = meta.data(), *mpos = mcu + B + 1, *mtoff = mpos + B, *mhd = mtoff + B + 1;
@@ -1243,14 +1131,11 @@ int attn_prefill_kv(const ApusHipAttnLayer *L, size_t B, const int32_t *cu, cons
     }
     memcpy(mcu, cu, (B + 1) * 4);
     memcpy(mpos, pos0, B * 4);
-    const bool half = fa_half_tiles(B, cu, pos0, L->nkv, is_short);
+    const bool half = fa_half_tiles(B, cu, pos0, L->nkv);
     const int32_t tq = half ? TQ16 : TQ;
     for (size_t s = 0; s < B; s++)
-        mtoff[s + 1] = mtoff[s] + (is_short(s) ? 0 : (cu[s + 1] - cu[s] + tq - 1) / tq);
+        mtoff[s + 1] = mtoff[s] + (cu[s + 1] - cu[s] + tq - 1) / tq;
     const size_t ntiles = (size_t)mtoff[B];
-    for (const Short &r : shorts)
-        if (int e = short_run(r, L, cu, pos0, rows, qg, k, v, kv, y)) return e;
-    if (ntiles == 0) return kOk;
     FaSeqs fs;
     fs.n = (int32_t)B;
     const int32_t *fdm = nullptr;

@@ -356,13 +356,8 @@ int apus_hip_attn_cache_unpack_paged(const ApusHipKvCache *kv, int32_t row,
  * Arguments as apus_hip_attn_decode with no limit on new tokens per
  * sequence (pos0[s] + new tokens <= max_seq). The attention runs as an
  * MFMA flash-attention kernel; y is a tolerance class of the reference
- * (|c - r| <= 2e-3 (|r| + sum_j |P_j V_j|)). A sequence of few new tokens
- * after a long prefix (512 positions and four times the new tokens, or
- * more) may run through the split-K decode kernels instead: the same class,
- * in another summation order (within the flash kernel a row's bits do not
- * depend on how a prompt is cut into calls or on the batch), and library
- * scratch of 4 KiB per 64 keys, kv head and 4 tokens. Supports d=256,
- * rot=64, nh=8*nkv. */
+ * (|c - r| <= 2e-3 (|r| + sum_j |P_j V_j|)). Supports d=256, rot=64,
+ * nh=8*nkv. */
 int apus_hip_attn_prefill(const ApusHipAttnLayer *L, size_t B,
                           const int32_t *cu, const int32_t *pos0,
                           const uint16_t *qg, const uint16_t *k,

@@ -141,14 +141,12 @@ def test_prefill_tile_edges(hip, orc):
 
 
 @pytest.mark.parametrize("lens,pos0", [
-    ([13], [1900]),                         # alone: no flash tile is left
-    ([40, 5, 13, 1, 0, 4, 200], [3, 2000, 1500, 512, 90, 3000, 700]),   # one run and a lone one
-    ([2, 300, 17], [2500, 64, 4000])])      # on either side of a prompt
+    ([13], [1900]),
+    ([40, 5, 13, 1, 0, 4, 200], [3, 2000, 1500, 512, 90, 3000, 700]),
+    ([2, 300, 17], [2500, 64, 4000])])
 def test_prefill_short_continuations(hip, orc, lens, pos0):
-    """Few new tokens after a long prefix, which run as pieces of 4 tokens
-    through the decode kernels beside the flash kernel's sequences: piece
-    remainders, an empty sequence among them, pieces of two sequences in
-    one call."""
+    """Few new tokens after a long prefix, alone and beside prompts, with an
+    empty sequence among them."""
     cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
     _run(hip, orc, np.random.default_rng(len(lens)), cu, pos0, 4032, tag="short")
 
@@ -184,36 +182,83 @@ def test_prefill_tile_sizes_agree(hip, orc, lens, pos0):
     assert torch.equal(y[:n], y1)
 
 
-def test_prefill_short_on_two_streams(hip):
-    """Short continuations keep their scratch in place and take turns where
-    the stream changes: the same bits on either stream, back to back."""
-    import torch
+def _continuations(hip, torch, rng, sizes, max_seq):
+    """Short continuations of different inputs: for each (tokens, cached
+    positions) the tokens, a function that packs a fresh cache and one that
+    runs the call on it."""
     dims = synth.ATTN_DIMS
     nh, nkv, d, rot, theta = dims
-    rng = np.random.default_rng(8)
-    n, p, max_seq = 13, 3000, 3040
     layer = hip.attn_layer(dims, {k: _td(torch, v) for k, v in synth.attn_weights(rng).items()})
-    t = {k: _td(torch, v) for k, v in synth.attn_tokens(rng, n).items()}
-    kc, vc = (_td(torch, synth.normal_bf16(rng, (p, nkv, d))) for _ in range(2))
-    ys, keep = [], []
+    calls = []
+    for n, p in sizes:
+        t = {k: _td(torch, v) for k, v in synth.attn_tokens(rng, n).items()}
+        kc, vc = (_td(torch, synth.normal_bf16(rng, (p, nkv, d))) for _ in range(2))
+        dk = torch.zeros((1, nkv, max_seq, d), dtype=torch.int16, device="cuda")
+        dv = torch.zeros((1, nkv, max_seq // 32, d, 32), dtype=torch.int16, device="cuda")
+        hip.attn_cache_pack(kc, vc, p, nkv, d, dk[0], dv[0], max_seq)
+        y = torch.zeros((n, nh * d), dtype=torch.int16, device="cuda")
+
+        def run(n=n, p=p, t=t, dk=dk, dv=dv, y=y):
+            hip.attn_prefill(layer, [0, n], [p], t["qg"], t["k"], t["v"], dk, dv, max_seq, y)
+        calls.append((run, y))
+    want = []
+    for run, y in calls:                    # one after the other
+        run()
+        torch.cuda.synchronize()
+        want.append(y.clone())
+        y.zero_()
     torch.cuda.synchronize()
+    assert not torch.equal(want[0][0], want[1][0])
+    return calls, want
+
+
+def test_prefill_short_on_two_streams(hip):
+    """Short continuations of different inputs on two streams, back to back
+    and unordered with each other: each gives what it gives alone (a prefill
+    keeps no intermediates that calls could share)."""
+    import torch
+    calls, want = _continuations(hip, torch, np.random.default_rng(8),
+                                 [(13, 3000), (9, 2500), (16, 3500), (5, 1700)], 3520)
     streams = [torch.cuda.Stream(), torch.cuda.Stream()]
     try:
-        for i in range(4):
-            hip.set_stream(streams[i % 2].cuda_stream)
-            with torch.cuda.stream(streams[i % 2]):
-                dk = torch.zeros((1, nkv, max_seq, d), dtype=torch.int16, device="cuda")
-                dv = torch.zeros((1, nkv, max_seq // 32, d, 32), dtype=torch.int16, device="cuda")
-                y = torch.zeros((n, nh * d), dtype=torch.int16, device="cuda")
-                hip.attn_cache_pack(kc, vc, p, nkv, d, dk[0], dv[0], max_seq)
-                hip.attn_prefill(layer, [0, n], [p], t["qg"], t["k"], t["v"], dk, dv, max_seq, y)
-            ys.append(y)
-            keep += [dk, dv]
+        for _ in range(8):
+            for i, (run, _y) in enumerate(calls):
+                hip.set_stream(streams[i % 2].cuda_stream)
+                run()
         torch.cuda.synchronize()
     finally:
         hip.set_stream(None)
-    for y in ys[1:]:
-        assert torch.equal(ys[0], y)
+    for (_, y), r in zip(calls, want):
+        assert torch.equal(y, r)
+
+
+def test_prefill_short_captured_beside_eager(hip):
+    """A short continuation captured into a graph and replayed on one stream
+    while an eager one of other inputs runs on the stream of the capture:
+    both give what they give alone, at every replay."""
+    import torch
+    calls, want = _continuations(hip, torch, np.random.default_rng(9), [(13, 3000), (9, 2500)],
+                                 3040)
+    (run0, y0), (run1, y1) = calls
+    cap, rep = torch.cuda.Stream(), torch.cuda.Stream()
+    try:
+        hip.set_stream(cap.cuda_stream)
+        run0()                              # on this stream before the capture
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=cap):
+            run0()
+        for _ in range(6):
+            y0.zero_()
+            y1.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(rep):
+                graph.replay()
+            run1()
+            torch.cuda.synchronize()
+            assert torch.equal(y0, want[0]) and torch.equal(y1, want[1])
+    finally:
+        hip.set_stream(None)
 
 
 def test_prefill_long(hip, orc):
@@ -256,7 +301,7 @@ def test_prefill_config3_vs_decode(hip):
     print(f"[attn_prefill config3] last rows vs decode {st}", flush=True)
 
 
-@pytest.mark.parametrize("T,cut", [(12, 7), (300, 173), (1000, 513)])
+@pytest.mark.parametrize("T,cut", [(12, 7), (300, 173), (1000, 513), (600, 597), (1913, 1900)])
 def test_prefill_split_equals_oneshot(hip, T, cut):
     """The reference's chunking invariance (its one-shot T=12 prefill must
     equal a 7 + 5 chunking bitwise, tests/m4c/README.md): T tokens
@@ -264,7 +309,8 @@ def test_prefill_split_equals_oneshot(hip, T, cut):
     starting at position `cut` over the cache the first filled) give the
     same outputs and the same cache, bit for bit. A row's scores, its
     running max / sum and its P.V run over keys 0..pos in the same 32-key
-    steps whichever call holds it."""
+    steps whichever call holds it, a few tokens after a long prefix among
+    them."""
     import torch
     dims = synth.ATTN_DIMS
     nh, nkv, d, rot, theta = dims
@@ -293,7 +339,10 @@ def test_prefill_split_equals_oneshot(hip, T, cut):
     assert torch.equal(y1, y2), "outputs"
 
 
-def test_prefill_batched_equals_alone(hip):
+@pytest.mark.parametrize("lens,pos0", [
+    ([37, 1, 64, 100], [0, 50, 31, 200]),
+    ([13, 4000, 5, 1], [1900, 0, 600, 3000])])    # few tokens after long prefixes
+def test_prefill_batched_equals_alone(hip, lens, pos0):
     """The reference's batch invariance (batched prefill == sequential,
     bitwise; tests/m9c): a ragged batch with cached prefixes and each
     sequence prefilled alone over its own cache give the same outputs and
@@ -302,10 +351,9 @@ def test_prefill_batched_equals_alone(hip):
     dims = synth.ATTN_DIMS
     nh, nkv, d, rot, theta = dims
     rng = np.random.default_rng(96)
-    lens, pos0 = [37, 1, 64, 100], [0, 50, 31, 200]
     cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
     B, T = len(lens), int(cu[-1])
-    max_seq = 320
+    max_seq = (max(p + n for n, p in zip(lens, pos0)) + 31) // 32 * 32
     w = synth.attn_weights(rng)
     tok = synth.attn_tokens(rng, T)
     kc = synth.normal_bf16(rng, (B, max_seq, nkv, d))
