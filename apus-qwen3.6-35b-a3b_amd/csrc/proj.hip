@@ -897,7 +897,9 @@ int launch_seq(const uint16_t *w, const uint16_t *x, uint16_t *y, size_t M, size
     if (int r = check_dims(M, O, K)) return r;
     if (M == 0 || O == 0) return kOk;
     if (M > 65535) return set_error(kErrUnsupported, "sequential gemm takes up to 65535 rows");
-    const bool vec = K % 8 == 0 && ((uintptr_t)w | (uintptr_t)x) % 16 == 0;
+    // (K = 0, zeros, has no pieces to load ahead and no rows per workgroup
+    // below: the scalar kernel, which reads nothing then)
+    const bool vec = K != 0 && K % 8 == 0 && ((uintptr_t)w | (uintptr_t)x) % 16 == 0;
     const dim3 grid(cdiv(O, 64), (unsigned)M);
     if (vec) {
         if (K * 2 > 64 * 1024) return set_error(kErrUnsupported, "sequential gemm takes K up to 32768");

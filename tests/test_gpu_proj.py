@@ -80,6 +80,19 @@ def test_gemm_dev_bitwise_chunks(hip, orc, M, O, K):
     assert np.array_equal(y.cpu().numpy().view(np.uint16), orc.bf16_gemm(w, x))
 
 
+@pytest.mark.parametrize("M,O", [(1, 1), (1, 130), (5, 64)])
+def test_gemm_empty_sums(hip, M, O):
+    """K = 0: every output is an empty sum, +0, and no operand is read."""
+    import torch
+    w, x = (torch.empty((n, 0), dtype=torch.int16, device="cuda") for n in (O, M))
+    y = torch.full((M, O), -1, dtype=torch.int16, device="cuda")
+    print(f"[proj] empty sums M={M} O={O}", flush=True)
+    hip.bf16_gemm_dev(w, x, y, exact=True)
+    torch.cuda.synchronize()
+    assert not y.cpu().any()
+    assert not hip.bf16_gemm(np.empty((O, 0), np.uint16), np.empty((M, 0), np.uint16)).any()
+
+
 def test_gemm_dev_bitwise_wide_range(hip, orc):
     """Operands whose magnitudes span 2^-60 .. 2^60 (every product still in
     fp32's normal range): the sequential kernel's fused multiply-add rounds
