@@ -233,10 +233,11 @@ __device__ __forceinline__ void split8(const float (&x)[8], u16x8 &hi, u16x8 &lo
 constexpr int CKP = DK + 8;            // bf16 row stride of the code copies
 
 // Two channels' 4-tap conv sums (tap order, one rounding per mul and add,
-// c/gdn.h:19-33; a product of bf16 values is exact in fp32, so the fused
-// form rounds where they do, products below 2^-126 aside), rounded to bf16
-// codes by one hardware round-to-nearest-even conversion
-// (v_cvt_pk_bf16_f32): the codes conv_sum4_code gives for finite sums.
+// c/gdn.h:19-33), rounded to bf16 codes by one hardware round-to-nearest-
+// even conversion (v_cvt_pk_bf16_f32): the codes conv_sum4_code gives for
+// finite sums. Not fused: a product below 2^-126 is not exact in fp32, and
+// added unrounded it can turn the sum's code (a layer call of 4096 tokens
+// 179.8 us, fused 178.7).
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t conv_sum4_pair(const float (&w0)[4], const float (&w1)[4],
@@ -244,13 +245,15 @@ __device__ __forceinline__ uint32_t conv_sum4_pair(const float (&w0)[4], const f
                                                    uint32_t x3) {
     auto lo = [](uint32_t v) { return __uint_as_float(v << 16); };
     auto hi = [](uint32_t v) { return __uint_as_float(v & 0xffff0000u); };
-    float a = fmaf(w0[0], lo(x0), 0.0f), c = fmaf(w1[0], hi(x0), 0.0f);
-    a = fmaf(w0[1], lo(x1), a);
-    c = fmaf(w1[1], hi(x1), c);
-    a = fmaf(w0[2], lo(x2), a);
-    c = fmaf(w1[2], hi(x2), c);
-    a = fmaf(w0[3], lo(x3), a);
-    c = fmaf(w1[3], hi(x3), c);
+    float a = 0.0f, c = 0.0f;
+    a = a + w0[0] * lo(x0);
+    c = c + w1[0] * hi(x0);
+    a = a + w0[1] * lo(x1);
+    c = c + w1[1] * hi(x1);
+    a = a + w0[2] * lo(x2);
+    c = c + w1[2] * hi(x2);
+    a = a + w0[3] * lo(x3);
+    c = c + w1[3] * hi(x3);
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, c}, bf16x2_t));
 }
 constexpr int TG = 16;                         // tokens per conv work item

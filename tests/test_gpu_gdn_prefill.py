@@ -120,6 +120,47 @@ def test_prefill_silu_every_code(hip, orc):
     assert err.max() <= 1e-4, float(err.max())
 
 
+def test_prefill_conv_small_products(hip, orc):
+    """The conv's products are rounded before they are added, as the
+    reference's are, also below 2^-126, where the product of two bf16 values
+    is not exact in fp32. Every v channel's taps give, with u = 2^-149,
+    32767 u, 1.5 u, 2^-110 and 2^-118: with 1.5 u rounded to 2 u first the
+    first two pass half an ulp of 2^-110, the sum lies above a bf16 tie and
+    the code is 2^-110 (1 + 2^-7); added unrounded they make 32768 u, both
+    ties go to even and the code is 2^-110. One token from a zero state, so
+    S = beta k v^T shows v to the chunk form's own 1e-5 against 2^-7."""
+    import torch
+    dims = synth.GDN_DIMS
+    hk, hv, dk, dv = dims
+    rng = np.random.default_rng(9)
+    kd = hk * dk
+    w = synth.gdn_weights(rng)
+    tok = synth.gdn_tokens(rng, 1)
+    conv, S = synth.gdn_state(rng, 1, zero=True)
+    taps = np.array([217.0, 3.0, 1.0, 1.0]) * np.exp2([-75.0, -75.0, -55.0, -59.0])
+    vals = np.array([151.0, 1.0, 1.0, 1.0]) * np.exp2([-74.0, -75.0, -55.0, -59.0])
+    w["conv_w"] = w["conv_w"].copy()
+    w["conv_w"].reshape(-1, 4)[2 * kd:] = synth.bf16_bits(taps.astype(np.float32))
+    x = synth.bf16_bits(vals.astype(np.float32))
+    conv.reshape(-1, 3)[2 * kd:] = x[:3]
+    tok["qkv"].reshape(-1)[2 * kd:] = x[3]
+    cu = np.array([0, 1], np.int32)
+    S_o = S.copy()
+    orc.gdn_mixer(dims, w, cu, tok["qkv"], tok["z"], tok["a"], tok["b"], conv.copy(), S_o)
+    layer = hip.gdn_layer(dims, {k: _dev(torch, v) for k, v in w.items()})
+    t = {k: _dev(torch, v) for k, v in tok.items()}
+    dS = torch.zeros((1, hv, dk, dv), device="cuda")
+    out = torch.empty_like(dS)
+    y = torch.empty((1, hv * dv), dtype=torch.int16, device="cuda")
+    hip.gdn_prefill(layer, cu, t["qkv"], t["z"], t["a"], t["b"], _dev(torch, conv), dS, y)
+    hip.gdn_state_unpack(dS, out)
+    torch.cuda.synchronize()
+    r = S_o.astype(np.float64)
+    assert np.abs(r).max() > 0.0
+    err = np.abs(out.cpu().numpy() - r).max(axis=2) / np.abs(r).max(axis=2)
+    assert err.max() <= 1e-4, float(err.max())
+
+
 def test_prefill_then_decode(hip, orc):
     """Prefill a prompt then decode one token from the device state: the
     state layout and conv state the prefill leaves are what decode reads."""
