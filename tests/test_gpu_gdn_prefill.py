@@ -82,13 +82,16 @@ def test_prefill_strong_decay(hip, orc):
                  a_scale=2.0, tag="strong_decay")
 
 
-def test_prefill_silu_every_code(hip, orc):
+@pytest.mark.parametrize("swap", [False, True])
+def test_prefill_silu_every_code(hip, orc, swap):
     """The chunk kernel's SiLU (from the table for one channel of a pair, by
     formula with the table behind it for the other) on every bf16 code of
-    magnitude 2^-80 .. 2^40 above -64 (below it the product goes to 0): 16 one-token sequences from a zero state, whose
-    conv passes the codes through (last tap 1). S = beta k v^T then, so
-    column j shows v_j = SiLU(code) to the chunk form's own 1e-5, against
-    2^-8 for a code that is one ulp off."""
+    magnitude 2^-80 .. 2^40 above -64 (below it the product goes to 0): 16
+    one-token sequences from a zero state, whose conv passes the codes
+    through (last tap 1); swap: with the two channels of every pair
+    exchanged, so that over both runs each code takes either way. S = beta k
+    v^T then, so column j shows v_j = SiLU(code) to the chunk form's own
+    1e-5, against 2^-8 for a code that is one ulp off."""
     import torch
     dims = synth.GDN_DIMS
     hk, hv, dk, dv = dims
@@ -102,6 +105,8 @@ def test_prefill_silu_every_code(hip, orc):
     exp = (codes >> 7) & 0xFF
     codes = np.where((exp >= 127 - 80) & (exp <= np.where(codes >> 15, 127 + 5, 127 + 40)), codes,
                      0x3F80)
+    if swap:
+        codes = np.ascontiguousarray(codes.reshape(-1, 2)[:, ::-1])
     tok["qkv"][:, 2 * kd:] = codes.reshape(B, hv * dv)
     conv, S = synth.gdn_state(rng, B, zero=True)
     cu = np.arange(B + 1, dtype=np.int32)
