@@ -1348,7 +1348,7 @@ int attn_decode_kv(const ApusHipAttnLayer *L, size_t B, const int32_t *cu, const
     auto launch = [&](auto nrb, const auto &m) {
         constexpr int NRB = decltype(nrb)::value, N = sizeof(m.pos0) / 4;
         if (total <= kFewKeys) {
-            APUS_TIMED("k_attn_scores",
+            APUS_TIMED("k_attn_scores_few",
                        k_attn_scores_few<NRB, N><<<(unsigned)nruns1, 256, 0, stream()>>>(
                            m, dmeta, qn, kv, (int)L->nh, (int)nkv, scale, As, st));
         } else {

@@ -1166,7 +1166,7 @@ int attn_prefill_kv(const ApusHipAttnLayer *L, size_t B, const int32_t *cu, cons
     const float scale = (float)(1.0 / sqrt((double)L->d));
     const ActTables *tabs = act_tables();
     if (!tabs) return kErrHip;
-    APUS_TIMED("k_attn_fa",
+    APUS_TIMED(half ? "k_attn_fa16" : "k_attn_fa",
                (half ? k_attn_fa16 : k_attn_fa)<<<(unsigned)(ntiles * L->nkv), 64 * NW, 0, stream()>>>(
                    fs, fdm, L->qn_w, rope, qg, kv, (int)L->nh, (int)L->nkv, scale, y, tabs->sig_bf,
                    attn_trace() ? attn_trace()->attno : nullptr));

@@ -77,7 +77,7 @@ int gdn_layer_run(const ApusHipGdnLayer *L, const ApusHipGdnProj *P, size_t B,
     in.w[1] = P->w_z;   in.y[1] = z;   in.ldy[1] = (int)vd;
     in.w[2] = P->w_b;   in.y[2] = b;   in.ldy[2] = (int)hv;
     in.w[3] = P->w_a;   in.y[3] = a;   in.ldy[3] = (int)hv;
-    if (int r = gemm_tile(in, ln1, T, H, "k_gemm_tile_in")) return r;
+    if (int r = gemm_tile(in, ln1, T, H, kGemmIn)) return r;
     const int rc = slot_in ? apus_hip_gdn_decode_slots(L, B, slot_in, slot_out, cu, qkv, z, a, b,
                                                        conv, S, y)
                            : apus_hip_gdn_decode(L, B, cu, qkv, z, a, b, conv, S, y);
@@ -86,7 +86,7 @@ int gdn_layer_run(const ApusHipGdnLayer *L, const ApusHipGdnProj *P, size_t B,
     out.n = 1;
     out.row0[1] = (int)H;
     out.w[0] = P->w_out; out.y[0] = ao; out.ldy[0] = (int)H;
-    return gemm_tile(out, y, T, vd, "k_gemm_tile_out");
+    return gemm_tile(out, y, T, vd, kGemmOut);
 }
 
 // The full-attention layer: wq | wk | wv -> mixer -> wo. rows: the paged
@@ -124,13 +124,13 @@ int attn_layer_run(const ApusHipAttnLayer *L, const ApusHipAttnProj *P, size_t B
     in.w[0] = P->wq; in.y[0] = qg; in.ldy[0] = (int)nq;
     in.w[1] = P->wk; in.y[1] = k;  in.ldy[1] = (int)nk;
     in.w[2] = P->wv; in.y[2] = v;  in.ldy[2] = (int)nk;
-    if (int r = gemm_tile(in, ln1, T, H, "k_gemm_tile_in")) return r;
+    if (int r = gemm_tile(in, ln1, T, H, kGemmIn)) return r;
     if (int r = attn_decode_kv(L, B, cu, pos0, rows, qg, k, v, kv, y)) return r;
     GemmSegs out{};
     out.n = 1;
     out.row0[1] = (int)H;
     out.w[0] = P->wo; out.y[0] = ao; out.ldy[0] = (int)H;
-    return gemm_tile(out, y, T, no, "k_gemm_tile_out");
+    return gemm_tile(out, y, T, no, kGemmOut);
 }
 
 }  // namespace

@@ -22,10 +22,13 @@ struct GemmSegs {
     int ldy[kMaxSegs];
 };
 
+// The product's place in a layer, which ends the timing / error name of its
+// launch: k_gemm_tile or k_gemm_wide, then nothing, _in or _out.
+enum GemmPlace { kGemmAlone = 0, kGemmIn, kGemmOut };
+
 // y = x w^T over the segments of sg (row0[n] output rows in all) for M rows
-// of x [M][K]; name: the timing / error name of the launch. Call
-// gemm_tile_check first.
-int gemm_tile(const GemmSegs &sg, const uint16_t *x, size_t M, size_t K, const char *name);
+// of x [M][K]. Call gemm_tile_check first.
+int gemm_tile(const GemmSegs &sg, const uint16_t *x, size_t M, size_t K, GemmPlace place);
 // K a multiple of 32, x 16-byte aligned, operands under 2 GiB (weights:
 // the caller checks their alignment)
 int gemm_tile_check(const uint16_t *x, size_t M, size_t O, size_t K);

@@ -786,9 +786,14 @@ __global__ __launch_bounds__(256) void k_gemm_reduce(GemmSegs sg, const float *_
     yr[3] = f2bf(sm.w);
 }
 
+// timing / error names by GemmPlace
+const char *const kTileNames[] = {"k_gemm_tile", "k_gemm_tile_in", "k_gemm_tile_out"};
+const char *const kWideNames[] = {"k_gemm_wide", "k_gemm_wide_in", "k_gemm_wide_out"};
+
 template <int WO, int WM, int TO, int TMM, int ST = kTileStages>
-int launch_tile(const GemmSegs &sg, const uint16_t *x, int M, int K, const char *name,
+int launch_tile(const GemmSegs &sg, const uint16_t *x, int M, int K, GemmPlace place,
                 int nsplit) {
+    const char *name = kTileNames[place];
     constexpr int BO = 32 * TO * WO, BM = 32 * TMM * WM;
     const int O = sg.row0[sg.n];
     const int nbo = (O + BO - 1) / BO, nbm = (M + BM - 1) / BM;
@@ -810,7 +815,8 @@ int launch_tile(const GemmSegs &sg, const uint16_t *x, int M, int K, const char 
 }
 
 template <int TO, int TMM, int ST>
-int launch_wide(const GemmSegs &sg, const uint16_t *x, int M, int K, const char *name) {
+int launch_wide(const GemmSegs &sg, const uint16_t *x, int M, int K, GemmPlace place) {
+    const char *name = kWideNames[place];
     constexpr int BO = 64 * TO, BM = 64 * TMM;
     const int O = sg.row0[sg.n], nbm = (M + BM - 1) / BM;
     const bool narrow = wide_narrow<TO>(O);
@@ -830,11 +836,11 @@ struct TileShape {
     int bo, bm;
     float one, fill, two;
     bool split;                             // has a K-split form
-    int (*run)(const GemmSegs &, const uint16_t *, int, int, const char *, int);
+    int (*run)(const GemmSegs &, const uint16_t *, int, int, GemmPlace, int);
 };
 template <int TO, int TMM, int ST>
-int run_wide(const GemmSegs &sg, const uint16_t *x, int M, int K, const char *nm, int) {
-    return launch_wide<TO, TMM, ST>(sg, x, M, K, nm);
+int run_wide(const GemmSegs &sg, const uint16_t *x, int M, int K, GemmPlace place, int) {
+    return launch_wide<TO, TMM, ST>(sg, x, M, K, place);
 }
 const TileShape kTileShapes[] = {
     {64, 64, 12.7f, 0.0f, 20.5f, true, launch_tile<2, 1, 1, 2>},
@@ -857,7 +863,7 @@ namespace apus {
 // split depends on M and K only, and every shape accumulates an element's
 // k16 steps in order, so a product's result is the same whichever shape
 // and launch (segmented or not) computes it.
-int gemm_tile(const GemmSegs &sg, const uint16_t *x, size_t M, size_t K, const char *nm) {
+int gemm_tile(const GemmSegs &sg, const uint16_t *x, size_t M, size_t K, GemmPlace place) {
     const int O = sg.row0[sg.n], cus = cu_count();
     const int nsplit = M <= 512 && K >= 4096 && O % 4 == 0 ? 2 : 1;
     const TileShape *best = nullptr;
@@ -876,7 +882,7 @@ int gemm_tile(const GemmSegs &sg, const uint16_t *x, size_t M, size_t K, const c
             tbest = us;
         }
     }
-    return best->run(sg, x, (int)M, (int)K, nm, nsplit);
+    return best->run(sg, x, (int)M, (int)K, place, nsplit);
 }
 
 // checks shared by the MFMA entry points: K a multiple of 32 (stages),
@@ -908,7 +914,7 @@ int launch_seq(const uint16_t *w, const uint16_t *x, uint16_t *y, size_t M, size
         // four, 16.8 with two), x rows as fp32 in at most 64 KiB of LDS
         const int R = (int)std::min<size_t>({M, 4, 16384 / K, cdiv(cdiv(O, 64) * M, cu_count())});
         if (K % kSeqK == 0 && R > 0)
-            APUS_TIMED("k_gemm_seq",
+            APUS_TIMED("k_gemm_seq64",
                        k_gemm_seq64<<<dim3(grid.x, cdiv(M, R)), 64 * (4 + R), R * K * 4, stream()>>>(
                            w, x, y, (int)M, (int)O, (int)K, R));
         else if (K * 4 <= 64 * 1024)
@@ -1011,7 +1017,7 @@ int apus_hip_bf16_gemm_mfma_dev(const uint16_t *w, const uint16_t *x, uint16_t *
     sg.w[0] = w;
     sg.y[0] = y;
     sg.ldy[0] = (int)O;
-    return gemm_tile(sg, x, M, K, "k_gemm_tile");
+    return gemm_tile(sg, x, M, K, kGemmAlone);
 }
 
 }  // extern "C"

@@ -695,9 +695,10 @@ def bench_mixed_block(torch, B, steps, warmup, seed, leg=None, proj=False):
         bytes_ += 3 * w_gdn + w_att + 4 * 2 * T * HID * 2
         flops_in = 2 * T * HID * (3 * (CD + VD + 2 * HV) + NH * 2 * AD + 2 * NKV * AD)
         flops_out = 2 * T * HID * (3 * VD + NH * AD)
-        table["k_gemm_tile_in"] = ("hbm", (3 * (CD + VD + 2 * HV) + NH * 2 * AD + 2 * NKV * AD)
+        for kern in ("k_gemm_tile", "k_gemm_wide"):        # the one that runs, by the shape
+            table[kern + "_in"] = ("hbm", (3 * (CD + VD + 2 * HV) + NH * 2 * AD + 2 * NKV * AD)
                                    * HID * 2 // 4 + T * HID * 2, HBM_PEAK)
-        table["k_gemm_tile_out"] = ("hbm", (3 * HID * VD + HID * NH * AD) * 2 // 4
+            table[kern + "_out"] = ("hbm", (3 * HID * VD + HID * NH * AD) * 2 // 4
                                     + T * HID * 2, HBM_PEAK)
     total, per, kt = time_steps(torch, step, steps, warmup, 1, table)
     st = float(np.mean(per))
@@ -859,10 +860,11 @@ def bench_proj(torch, M, exact, steps, warmup, seed):
         w, x, y = sets[i]
         apus_hip.bf16_gemm_dev(w, x, y, exact=exact)
 
-    kname = "k_gemm_seq" if exact else "k_gemm_tile"
+    knames = ("k_gemm_seq64",) if exact else ("k_gemm_tile", "k_gemm_wide")
     bytes_ = O * K * 2 + M * K * 2 + M * O * 2
     flops = 2 * M * O * K
-    table = {kname: ("hbm", bytes_, HBM_PEAK) if M <= 256 else ("mfma", flops, BF16_PEAK)}
+    table = {k: ("hbm", bytes_, HBM_PEAK) if M <= 256 else ("mfma", flops, BF16_PEAK)
+             for k in knames}                              # the one that runs, by the shape
     total, per, kt = time_steps(torch, step, steps, warmup, nsets, table)
     wl = f"gdn_in_proj_m{M}"
     return dict(workload=wl, tokens_per_step=M, ms_per_step=total / steps * 1e3,
