@@ -113,11 +113,17 @@ def test_decode_few_and_ring_kernels_agree(hip):
     keys = lambda n: hip.attn_split_check(cu[:n + 1], pos0[:n])["writer_groups"] * 64
     assert keys(B - 1) <= 8192 * 64 < keys(B)
     ys = []
-    for n in (B - 1, B):
-        y = torch.zeros((int(cu[n]), nh * d), dtype=torch.bfloat16, device=dev)
-        hip.attn_decode_paged(layer, np.arange(n), cu[:n + 1], pos0[:n], t["qg"], t["k"], t["v"], kv, y)
-        ys.append(y[:int(cu[B - 1])].double())
+    hip.timing_enable(True)
+    try:
+        for n in (B - 1, B):
+            y = torch.zeros((int(cu[n]), nh * d), dtype=torch.bfloat16, device=dev)
+            hip.attn_decode_paged(layer, np.arange(n), cu[:n + 1], pos0[:n], t["qg"], t["k"], t["v"], kv, y)
+            ys.append(y[:int(cu[B - 1])].double())
+        ran = [hip.timing_get(k)[1] for k in ("k_attn_scores_few", "k_attn_scores")]
+    finally:
+        hip.timing_enable(False)
     torch.cuda.synchronize()
+    assert ran == [1, 1]
     assert torch.isfinite(ys[0]).all()
     assert float((ys[0] - ys[1]).norm() / ys[1].norm()) <= 2e-3
 

@@ -174,10 +174,18 @@ def test_prefill_tile_sizes_agree(hip, orc, lens, pos0):
                         dk[0], dv[0], max_seq)
     dk1, dv1 = dk[:1].clone(), dv[:1].clone()
     y = torch.empty((n + fill, nh * d), dtype=torch.int16, device="cuda")
-    hip.attn_prefill(layer, [0, n, n + fill], [p, 0], t["qg"], t["k"], t["v"], dk, dv, max_seq, y)
     y1 = torch.empty((n, nh * d), dtype=torch.int16, device="cuda")
-    hip.attn_prefill(layer, [0, n], [p], t["qg"][:n], t["k"][:n], t["v"][:n], dk1, dv1, max_seq, y1)
+    hip.timing_enable(True)
+    try:
+        hip.attn_prefill(layer, [0, n, n + fill], [p, 0], t["qg"], t["k"], t["v"], dk, dv, max_seq,
+                         y)
+        hip.attn_prefill(layer, [0, n], [p], t["qg"][:n], t["k"][:n], t["v"][:n], dk1, dv1,
+                         max_seq, y1)
+        ran = [hip.timing_get(k)[1] for k in ("k_attn_fa", "k_attn_fa16")]
+    finally:
+        hip.timing_enable(False)
     torch.cuda.synchronize()
+    assert ran == [1, 1]
     assert torch.equal(dk[0], dk1[0]) and torch.equal(dv[0], dv1[0])
     assert torch.equal(y[:n], y1)
 

@@ -113,13 +113,13 @@ def test_gemm_dev_bitwise_wide_range(hip, orc):
     assert np.array_equal(hip.bf16_gemv(w, np.ascontiguousarray(x[0])), orc.bf16_gemm(w, x)[0])
 
 
-# one shape per tile configuration of the MFMA GEMM (64 x 64, 128 x 128,
-# 128 x 256, 256 x 256), with ragged row / output edges and an output count
-# that is not a multiple of 4 (the element-store epilogue)
+# from one tile to most of a chip of them, with ragged row / output
+# edges, a split K, and an output count that is not a multiple of 4 (the
+# element-store epilogue)
 @pytest.mark.parametrize("M,O,K", [(64, 12352, 2048), (200, 1000, 4096), (1, 70, 32),
-                                   (300, 5000, 512),    # 128 x 128 tiles
-                                   (260, 10240, 256),   # 128 x 256 tiles
-                                   (1000, 1000, 512),   # 256 x 256, ragged edges
+                                   (300, 5000, 512),
+                                   (260, 10240, 256),
+                                   (1000, 1000, 512),   # ragged edges
                                    (700, 517, 64)])     # O % 4 != 0
 def test_gemm_mfma_tolerance(hip, orc, M, O, K):
     import torch
