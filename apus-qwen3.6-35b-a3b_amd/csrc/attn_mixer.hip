@@ -1199,8 +1199,8 @@ constexpr size_t kFewKeys = (size_t)8192 * 64;
 // per streaming wavefront of one round of resident workgroups, or two per CU
 // for k_attn_scores_few (every run costs P.V a statistic: one sequence at
 // 60,000 positions 57 us with two, 92 with eleven). P.V: three runs per CU
-// of two wavefronts each, two while that leaves runs of 256 keys or less (each
-// run writes 8 KiB of partials per row block, so more runs cost more than
+// of two wavefronts each, or two (then of up to 384 keys) where three would
+// be of 256 keys or less (each run writes 8 KiB of partials per row block, so more runs cost more than
 // the wavefronts they add: 64 sequences at 32768 positions, P.V 351 us with
 // three runs per CU, 368 with six).
 static void attn_split_sizes(size_t total, size_t max_tok, size_t cus, int32_t *T1, int32_t *T2) {

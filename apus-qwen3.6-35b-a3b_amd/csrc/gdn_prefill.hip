@@ -302,7 +302,8 @@ __device__ __forceinline__ void conv_rows16(const uint16_t *__restrict__ qkv, si
 // outside [2^-60, 16]. A gather of 64 random codes keeps the address unit
 // busy about as long as the formula keeps the VALU, so one of each per pair
 // runs on both (4096 tokens: WY 81.6 us with every code gathered, 81.9 with
-// every code by the formula, 75.8 so). f1: bit TG - 1 - j: code j in doubt.
+// every code by the formula, 75.8 so; each about 1 us less than with the
+// sums above unfused). f1: bit TG - 1 - j: code j in doubt.
 __device__ __forceinline__ void conv_codes16(const ConvRows &R, int tg, int nt,
                                              const uint16_t *__restrict__ silu_bf,
                                              uint16_t (&c0)[TG], uint16_t (&c1)[TG]) {
@@ -709,7 +710,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
 // XCDs) and so share its L2. Longest first: a long sequence's slices walk
 // their chunks one after the other, and started behind the short ones' they
 // ran on alone at the end (lengths 997, 5, 43, 13, 65, 75, slices of a
-// sequence spread over the grid: 75 us; longest first 45).
+// sequence spread over the grid: 75 us; longest first 52).
 // 512 threads in two roles, two wavefronts per SIMD:
 //   waves 0-3 carry the recurrence: D = U - W S0 (rows 16w..), then
 //             S1^T = G_C S0^T + Dp^T K (state rows 32w..);

@@ -160,8 +160,9 @@ __global__ __launch_bounds__(64) void k_gemm_seq(const uint16_t *__restrict__ w,
 // the sum before it, its loads are 16-byte pieces of 64 rows, and the weights
 // are read once per row. 12352 x 2048: one row 18.0 -> 16.3 us, 3 rows 30.2 ->
 // 19.5, 8 rows 72 -> 31; 2048 x 4096 33.1 -> 27.2. What is left is the chain:
-// 6 ns a k (reads placed between its multiply-adds, or a part ahead of them,
-// made that 6.5 to 6.9).
+// 6 ns a k, where a dependent add alone takes 4 and each chunk adds its
+// barrier and the wait for its first reads (reads placed between the
+// multiply-adds, or a part ahead of them, made it 6.5 to 6.9).
 constexpr int kSeqK = 64;                  // k per chunk
 constexpr int kSeqDepth = 8;               // chunks in flight per loader
 __global__ __launch_bounds__(512) void k_gemm_seq64(const uint16_t *__restrict__ w,
@@ -860,9 +861,10 @@ namespace apus {
 // The shape with the least estimated time. Decode-sized row counts with a
 // long K (the output projections, K = 4096) split K in two: twice the
 // workgroups for the few output tiles (w_out at 325 rows: 27 -> 21 us). The
-// split depends on M and K only, and every shape accumulates an element's
-// k16 steps in order, so a product's result is the same whichever shape
-// and launch (segmented or not) computes it.
+// split depends on M, K and whether the launch's outputs are a multiple of 4,
+// and every shape accumulates an element's k16 steps in order, so a product's
+// result is the same whichever shape computes it, and segmented or not where
+// the launches agree on that.
 int gemm_tile(const GemmSegs &sg, const uint16_t *x, size_t M, size_t K, GemmPlace place) {
     const int O = sg.row0[sg.n], cus = cu_count();
     const int nsplit = M <= 512 && K >= 4096 && O % 4 == 0 ? 2 : 1;
